@@ -1303,6 +1303,7 @@ hipError_t launch_prefill_attention(const PrefillAttnArgs& a, KvDtype kv, hipStr
   if (a.out_split.hi && (!a.out_split.lo || !a.out_split.inv || a.out_split.chunk != kSplitChunkFine ||
                          a.d % kSplitChunkFine != 0))
     return hipErrorInvalidValue;
+  if (kv == kKvF16 && prefill_attention_many_rows(a)) return launch_prefill_attention_many_rows(a, stream);
   return kv == kKvF16 ? launch_prefill_attention_kv<__half>(a, stream)
                       : launch_prefill_attention_kv<float>(a, stream);
 }

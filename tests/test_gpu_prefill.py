@@ -139,6 +139,38 @@ def test_prefill_attention_group_sizes(gpu, oracle, hq, hkv):
         assert rel_err(got[t], ref) < TOL, t
 
 
+@pytest.mark.parametrize("d", [32, 64, 96])
+@pytest.mark.parametrize("hq,hkv,start,T", [(16, 2, 0, 449), (16, 2, 37, 480), (8, 2, 1000, 641), (8, 4, 511, 930),
+                                            (12, 2, 20, 1300)])
+def test_prefill_attention_many_rows(gpu, d, hq, hkv, start, T):
+    # the 32-query kernel: a last query tile of 1, 32, 1, 2 and 20 rows, groups
+    # of 8, 4, 2 and 6 heads, key ranges of unequal length, a context that
+    # crosses segments.  Against 64 bits:
+    # q and p carry 22 bits (2.4e-7), sums are fp32 over at most 1,641 keys of
+    # like size (random rounding, some 40 ulp of the sum at most): 1e-5 of the
+    # largest value, where one wrong key among 1,641 is about 1e-2.
+    mmr = gpu
+    print(f"[case] prefill attention many rows d={d} hq={hq} hkv={hkv} start={start} T={T}", flush=True)
+    rng = np.random.default_rng(d + hq + start + T)
+    n = start + T
+    k = rng.standard_normal((hkv, n, d)).astype(np.float16)
+    v = rng.standard_normal((hkv, n, d)).astype(np.float16)
+    q = (2 * rng.standard_normal((T, hq * d))).astype(np.float32)
+    cache = mmr.KvCache(hkv, d, n, mmr.KV_F16)
+    cache.upload(k, v)
+    dq, out = mmr.DeviceArray.from_numpy(q), mmr.DeviceArray((T, hq * d), np.float32)
+    mmr.prefill_attention(dq, cache, start, T, hq, hkv, d, out)
+    got = out.numpy().reshape(T, hq, d)
+    hidden = np.arange(n)[None, :] > start + np.arange(T)[:, None]
+    for h in range(hq):
+        g = h // (hq // hkv)
+        s = q.reshape(T, hq, d)[:, h].astype(np.float64) @ k[g].astype(np.float64).T / np.sqrt(d)
+        s[hidden] = -np.inf
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        ref = p @ v[g].astype(np.float64) / p.sum(axis=1, keepdims=True)
+        assert rel_err(got[:, h], ref) < 1e-5, h
+
+
 def synth_model(mmr, g):
     return mmr.Model.synthetic(mmr.make_config(**g["config"]), g["seed"], g["std"], g["round_fp16"])
 
