@@ -467,7 +467,7 @@ def batched_decode(mmr, model, batch: int, prompt_len: int, context: int) -> dic
     step_ms = np.array([ev[i + 1].elapsed_ms(ev[i + 2]) for i in range(steps)])
     decode_ms = ev[1].elapsed_ms(ev[-1])
     out = {"batch": batch, "prompt_tokens": prompt_len, "context": context, "kv_cache": "f16 paged (64-token pages)",
-           "prefill_ms": round(ev[0].elapsed_ms(ev[1]), 2), "prefill_mode": "batched decode steps over the prompts",
+           "prefill_ms": round(ev[0].elapsed_ms(ev[1]), 2), "prefill_mode": "prefill layers over all prompts' rows but the last, then batched steps",
            "decode_steps": steps, "decode_ms": round(decode_ms, 2),
            "aggregate_tok_s": round(batch * steps / (decode_ms * 1e-3), 1),
            "p50_step_ms": round(float(np.median(step_ms)), 4), "p90_step_ms": round(float(np.percentile(step_ms, 90)), 4),

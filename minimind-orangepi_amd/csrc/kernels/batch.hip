@@ -27,6 +27,18 @@ __global__ __launch_bounds__(kBatchThreads) void batch_embed_kernel(const __half
     h[static_cast<int64_t>(b) * hidden + i] = __half2float(row[i]);
 }
 
+// Embedding rows of tokens first .. first + tokens - 1 of each sequence.
+__global__ __launch_bounds__(kBatchThreads) void batch_embed_rows_kernel(const __half* embed, const int32_t* seq,
+                                                                         int seq_stride, int first, int tokens,
+                                                                         int vocab, int hidden, float* h) {
+  const int r = blockIdx.x, b = r / tokens;
+  int token = seq[static_cast<int64_t>(b) * seq_stride + first + r % tokens];
+  token = token < 0 ? 0 : (token >= vocab ? vocab - 1 : token);
+  const __half* row = embed + static_cast<int64_t>(token) * hidden;
+  for (int i = threadIdx.x; i < hidden; i += kBatchThreads)
+    h[static_cast<int64_t>(r) * hidden + i] = __half2float(row[i]);
+}
+
 // First-index argmax of one sequence's logits (std::max_element,
 // language_model.cpp:408-413) and the step bookkeeping.
 __global__ __launch_bounds__(kBatchThreads) void batch_argmax_kernel(const float* logits, int vocab,
@@ -624,6 +636,14 @@ hipError_t launch_batch_embed(const __half* embed, const int32_t* seq, int seq_s
   if (batch <= 0 || hidden <= 0) return hipErrorInvalidValue;
   const dim3 grid((hidden + kBatchThreads - 1) / kBatchThreads, batch);
   batch_embed_kernel<<<grid, kBatchThreads, 0, stream>>>(embed, seq, seq_stride, pos, vocab, hidden, h);
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_embed_rows(const __half* embed, const int32_t* seq, int seq_stride, int first, int tokens,
+                                   int batch, int vocab, int hidden, float* h, hipStream_t stream) {
+  if (batch <= 0 || tokens <= 0 || hidden <= 0 || first < 0 || first + tokens > seq_stride) return hipErrorInvalidValue;
+  batch_embed_rows_kernel<<<static_cast<unsigned>(batch * tokens), kBatchThreads, 0, stream>>>(
+      embed, seq, seq_stride, first, tokens, vocab, hidden, h);
   return hipGetLastError();
 }
 

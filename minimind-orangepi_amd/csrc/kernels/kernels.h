@@ -340,6 +340,19 @@ bool gemm_presplit_supported(int m, int n, int k);
 bool gemm_swiglu_split_supported(int m, int n, int k);
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
 
+// A batch's KV page pools ([page][Hkv][kKvPage][D], see AttnArgs): page p of
+// sequence b is physical page p * interleave + b.  k = nullptr: none.
+struct KvPool {
+  void* k = nullptr;
+  void* v = nullptr;
+  int interleave = 0;
+};
+// Element offset of sequence b's row for token t and KV head g.
+__host__ __device__ constexpr int64_t kv_pool_offset(int interleave, int b, int t, int g, int hkv, int d) {
+  const int64_t page = static_cast<int64_t>(t / kKvPage) * interleave + b;
+  return ((page * hkv + g) * kKvPage + t % kKvPage) * d;
+}
+
 // Rows of the fused qkv projection for tokens at positions start ..
 // start + tokens - 1: per-head q/k RMSNorm + RoPE, q -> query rows, k/v
 // written to cache rows row0 .. row0 + tokens - 1 (row0 = start when cache
@@ -362,6 +375,10 @@ struct QkvRowsArgs {
   int hq = 0, hkv = 0, d = 0;
   float* query = nullptr;  // [tokens][query_stride]
   int query_stride = 0;
+  // A batch: `tokens` rows of each of `seqs` sequences, all from the same
+  // start; sequence b's rows are b * tokens .. and its cache rows go to the pool.
+  int seqs = 1;
+  KvPool pool;
 };
 constexpr int kQkvRowsMaxParts = 4;
 hipError_t launch_qkv_rows(const QkvRowsArgs& a, KvDtype kv, hipStream_t stream);
@@ -380,6 +397,10 @@ struct PrefillAttnArgs {
   // Optional: the output also as SplitPlanes with kSplitChunkFine chunks,
   // planes [tokens][out_stride], inv [tokens][hq d / 32]; needs d % 32 == 0.
   SplitPlanes out_split;
+  // A batch, as in QkvRowsArgs: rows b * tokens .. of query and out are
+  // sequence b's, its keys and values in the pool.
+  int seqs = 1;
+  KvPool pool;
 };
 hipError_t launch_prefill_attention(const PrefillAttnArgs& a, KvDtype kv, hipStream_t stream);
 // The kernel for many rows of an fp16 cache (prefill_attention.hip), which
@@ -394,6 +415,9 @@ hipError_t launch_prefill_attention_many_rows(const PrefillAttnArgs& a, hipStrea
 // (the host validates every id it uploads).
 hipError_t launch_batch_embed(const __half* embed, const int32_t* seq, int seq_stride, const int32_t* pos, int batch,
                               int vocab, int hidden, float* h, hipStream_t stream);
+// h[b * tokens + t][:] = embed[seq[b][first + t]], t < tokens.
+hipError_t launch_batch_embed_rows(const __half* embed, const int32_t* seq, int seq_stride, int first, int tokens,
+                                   int batch, int vocab, int hidden, float* h, hipStream_t stream);
 // Per sequence: first index of the maximum of logits[b][:vocab]; token_out[b]
 // receives it, and the step bookkeeping of launch_argmax_finalize runs per
 // sequence (seq[b][p + 1] when p + 1 >= prompt_len[b], then pos[b] = p + 1).

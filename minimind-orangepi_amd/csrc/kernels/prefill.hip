@@ -680,7 +680,7 @@ __global__ __launch_bounds__(kWave* kSkinnyWaves) void gemm_skinny_kernel(GemmAr
 // token); a block holds kQkvRowsTokens consecutive tokens of one head, grid
 // (hq + hkv, ceil(tokens / kQkvRowsTokens)).
 constexpr int kQkvRowsTokens = 4;
-template <typename KV, int D>
+template <typename KV, int D, bool kPool>
 __global__ __launch_bounds__(kWave* kQkvRowsTokens) void qkv_rows_kernel(QkvRowsArgs a) {
   __shared__ float x_all[kQkvRowsTokens][D];
   const int b = blockIdx.x;
@@ -692,10 +692,11 @@ __global__ __launch_bounds__(kWave* kQkvRowsTokens) void qkv_rows_kernel(QkvRows
   const int t_raw = blockIdx.y * kQkvRowsTokens + wave;
   const bool live = t_raw < a.tokens;
   const int t = min(t_raw, a.tokens - 1);
+  const int64_t out_row = (kPool ? static_cast<int64_t>(blockIdx.z) * a.tokens : 0) + t;  // blockIdx.z: sequence of a batch
   float* x_s = x_all[wave];
   const bool is_q = b < a.hq;
   const int head = is_q ? b : b - a.hq;
-  const float* row = a.qkv + static_cast<int64_t>(t) * a.qkv_stride;
+  const float* row = a.qkv + out_row * a.qkv_stride;
   const float* src = row + (is_q ? head * D : a.hq * D + head * D);
   const float* vsrc = row + a.hq * D + a.hkv * D + head * D;
   const float* w = is_q ? a.q_norm : a.k_norm;
@@ -746,14 +747,15 @@ __global__ __launch_bounds__(kWave* kQkvRowsTokens) void qkv_rows_kernel(QkvRows
   __syncthreads();
   if (!live) return;
   if (is_q) {
-    float* dst = a.query + static_cast<int64_t>(t) * a.query_stride + head * D;
+    float* dst = a.query + out_row * a.query_stride + head * D;
     for (int i = lane; i < D; i += kWave) dst[i] = x_s[i];
   } else {
     const int row = a.row0 + t;
-    const int seg = kv_segment(row);
-    const int64_t off = kv_segment_offset(seg, row, head, a.hkv, D);
-    KV* kdst = static_cast<KV*>(a.seg.s[seg].k) + off;
-    KV* vdst = static_cast<KV*>(a.seg.s[seg].v) + off;
+    const int seg = kPool ? 0 : kv_segment(row);
+    const int64_t off = kPool ? kv_pool_offset(a.pool.interleave, blockIdx.z, row, head, a.hkv, D)
+                              : kv_segment_offset(seg, row, head, a.hkv, D);
+    KV* kdst = static_cast<KV*>(kPool ? a.pool.k : a.seg.s[seg].k) + off;
+    KV* vdst = static_cast<KV*>(kPool ? a.pool.v : a.seg.s[seg].v) + off;
     if (lane < D) {
       kdst[lane] = from_float<KV>(x_s[lane]);
       vdst[lane] = from_float<KV>(v0);
@@ -799,7 +801,7 @@ struct PrefillTileRegs {
   uint4 k[kPer], v[kPer];
 };
 
-template <typename KV, int D>
+template <typename KV, int D, bool kPool>
 __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel(PrefillAttnArgs a) {
   using Regs = PrefillTileRegs<KV, D>;
   constexpr int CH = Regs::CH;
@@ -821,7 +823,8 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel
   const int lane = threadIdx.x % kWave;
   const int q0 = blockIdx.x * kPrefillQueries;
   const int qi = lane % 16, kq = lane / 16;  // query column, k slot
-  const int qrow = min(q0 + qi, a.tokens - 1);
+  const int64_t row0 = kPool ? static_cast<int64_t>(blockIdx.z) * a.tokens : 0;  // blockIdx.z: sequence of a batch
+  const int64_t qrow = row0 + min(q0 + qi, a.tokens - 1);
   const int qpos = a.start + q0 + qi;
   float* k_s = stage[wave];            // [KT][LD]
   float* v_s = stage[wave] + KT * LD;  // [KT][LD]
@@ -841,10 +844,11 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel
   // one head's rows are contiguous: one segment lookup per tile.
   auto fetch = [&](int tile, Regs& r) {
     const int t0 = tile * KT;
-    const int seg = kv_segment(t0);
-    const int64_t tile_off = kv_segment_offset(seg, t0, g, a.hkv, D);
-    const KV* ktile = static_cast<const KV*>(a.seg.s[seg].k) + tile_off;
-    const KV* vtile = static_cast<const KV*>(a.seg.s[seg].v) + tile_off;
+    const int seg = kPool ? 0 : kv_segment(t0);
+    const int64_t tile_off = kPool ? kv_pool_offset(a.pool.interleave, blockIdx.z, t0, g, a.hkv, D)
+                                   : kv_segment_offset(seg, t0, g, a.hkv, D);
+    const KV* ktile = static_cast<const KV*>(kPool ? a.pool.k : a.seg.s[seg].k) + tile_off;
+    const KV* vtile = static_cast<const KV*>(kPool ? a.pool.v : a.seg.s[seg].v) + tile_off;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int c = min(lane + i * kWave, kChunks - 1);
@@ -866,7 +870,7 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel
   const float qscale = 1.4426950408889634f / sqrtf(static_cast<float>(D));
   float4 qf[kF16 ? 1 : DT];
   uint4 qh[kF16 ? D / 32 : 1], ql[kF16 ? D / 32 : 1];  // f16x8 bits
-  const float* qsrc = a.query + static_cast<int64_t>(qrow) * a.query_stride + h * D;
+  const float* qsrc = a.query + qrow * a.query_stride + h * D;
   if constexpr (kF16) {
 #pragma unroll
     for (int j = 0; j < D / 32; ++j) {
@@ -1065,7 +1069,7 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel
     float o = 0.0f;
 #pragma unroll
     for (int w = 0; w < kPrefillWaves; ++w) o = fmaf(o_sh[(w * D + dim) * kMergeLd + q], m_sh[w * kPrefillQueries + q], o);
-    const int64_t off = static_cast<int64_t>(q0 + q) * a.out_stride + h * D + dim;
+    const int64_t off = (row0 + q0 + q) * a.out_stride + h * D + dim;
     if (a.out && valid) a.out[off] = o;
     if constexpr (D % kSplitChunkFine == 0) {
       if (a.out_split.hi) {
@@ -1081,7 +1085,7 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel
           __builtin_memcpy(a.out_split.hi + off, &hh, 2);
           __builtin_memcpy(a.out_split.lo + off, &ll, 2);
           if (dim % kSplitChunkFine == 0)
-            a.out_split.inv[static_cast<int64_t>(q0 + q) * (a.hq * D / kSplitChunkFine) + (h * D + dim) / kSplitChunkFine] =
+            a.out_split.inv[(row0 + q0 + q) * (a.hq * D / kSplitChunkFine) + (h * D + dim) / kSplitChunkFine] =
                 ldexpf(1.0f, e - 15);
         }
       }
@@ -1158,31 +1162,31 @@ hipError_t launch_gemm_any(const GemmArgs& g, hipStream_t s) {
   }
 }
 
-template <typename KV>
+template <typename KV, bool kPool>
 hipError_t launch_qkv_rows_kv(const QkvRowsArgs& a, hipStream_t s) {
-  const dim3 grid(a.hq + a.hkv, (a.tokens + kQkvRowsTokens - 1) / kQkvRowsTokens);
+  const dim3 grid(a.hq + a.hkv, (a.tokens + kQkvRowsTokens - 1) / kQkvRowsTokens, a.seqs);
   const dim3 block(kWave * kQkvRowsTokens);
   switch (a.d) {
-    case 16: qkv_rows_kernel<KV, 16><<<grid, block, 0, s>>>(a); break;
-    case 32: qkv_rows_kernel<KV, 32><<<grid, block, 0, s>>>(a); break;
-    case 64: qkv_rows_kernel<KV, 64><<<grid, block, 0, s>>>(a); break;
-    case 96: qkv_rows_kernel<KV, 96><<<grid, block, 0, s>>>(a); break;
-    case 128: qkv_rows_kernel<KV, 128><<<grid, block, 0, s>>>(a); break;
+    case 16: qkv_rows_kernel<KV, 16, kPool><<<grid, block, 0, s>>>(a); break;
+    case 32: qkv_rows_kernel<KV, 32, kPool><<<grid, block, 0, s>>>(a); break;
+    case 64: qkv_rows_kernel<KV, 64, kPool><<<grid, block, 0, s>>>(a); break;
+    case 96: qkv_rows_kernel<KV, 96, kPool><<<grid, block, 0, s>>>(a); break;
+    case 128: qkv_rows_kernel<KV, 128, kPool><<<grid, block, 0, s>>>(a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-template <typename KV>
+template <typename KV, bool kPool>
 hipError_t launch_prefill_attention_kv(const PrefillAttnArgs& a, hipStream_t s) {
-  const dim3 grid((a.tokens + kPrefillQueries - 1) / kPrefillQueries, a.hq);
+  const dim3 grid((a.tokens + kPrefillQueries - 1) / kPrefillQueries, a.hq, a.seqs);
   const dim3 block(kWave * kPrefillWaves);
   switch (a.d) {
-    case 16: prefill_attention_kernel<KV, 16><<<grid, block, 0, s>>>(a); break;
-    case 32: prefill_attention_kernel<KV, 32><<<grid, block, 0, s>>>(a); break;
-    case 64: prefill_attention_kernel<KV, 64><<<grid, block, 0, s>>>(a); break;
-    case 96: prefill_attention_kernel<KV, 96><<<grid, block, 0, s>>>(a); break;
-    case 128: prefill_attention_kernel<KV, 128><<<grid, block, 0, s>>>(a); break;
+    case 16: prefill_attention_kernel<KV, 16, kPool><<<grid, block, 0, s>>>(a); break;
+    case 32: prefill_attention_kernel<KV, 32, kPool><<<grid, block, 0, s>>>(a); break;
+    case 64: prefill_attention_kernel<KV, 64, kPool><<<grid, block, 0, s>>>(a); break;
+    case 96: prefill_attention_kernel<KV, 96, kPool><<<grid, block, 0, s>>>(a); break;
+    case 128: prefill_attention_kernel<KV, 128, kPool><<<grid, block, 0, s>>>(a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1291,21 +1295,29 @@ hipError_t launch_gemm(const GemmArgs& g, hipStream_t s) {
 }
 
 hipError_t launch_qkv_rows(const QkvRowsArgs& a, KvDtype kv, hipStream_t stream) {
-  if (!attention_supported(a.hq, a.hkv, a.d) || a.tokens <= 0 || a.qkv_parts < 1 ||
-      a.qkv_parts > kQkvRowsMaxParts || (a.qkv_parts > 1 && a.qkv_part_stride < int64_t{a.tokens} * a.qkv_stride))
+  if (!attention_supported(a.hq, a.hkv, a.d) || a.tokens <= 0 || a.qkv_parts < 1 || a.seqs < 1 ||
+      a.qkv_parts > kQkvRowsMaxParts ||
+      (a.qkv_parts > 1 && a.qkv_part_stride < int64_t{a.seqs} * a.tokens * a.qkv_stride))
     return hipErrorInvalidValue;
-  return kv == kKvF16 ? launch_qkv_rows_kv<__half>(a, stream) : launch_qkv_rows_kv<float>(a, stream);
+  if (a.pool.k ? (!a.pool.v || a.pool.interleave < a.seqs) : a.seqs != 1) return hipErrorInvalidValue;
+  if (a.pool.k)
+    return kv == kKvF16 ? launch_qkv_rows_kv<__half, true>(a, stream) : launch_qkv_rows_kv<float, true>(a, stream);
+  return kv == kKvF16 ? launch_qkv_rows_kv<__half, false>(a, stream) : launch_qkv_rows_kv<float, false>(a, stream);
 }
 
 hipError_t launch_prefill_attention(const PrefillAttnArgs& a, KvDtype kv, hipStream_t stream) {
-  if (!attention_supported(a.hq, a.hkv, a.d) || a.tokens <= 0 || a.start < 0) return hipErrorInvalidValue;
+  if (!attention_supported(a.hq, a.hkv, a.d) || a.tokens <= 0 || a.start < 0 || a.seqs < 1) return hipErrorInvalidValue;
+  if (a.pool.k ? (!a.pool.v || a.pool.interleave < a.seqs) : a.seqs != 1) return hipErrorInvalidValue;
   if (!a.out && !a.out_split.hi) return hipErrorInvalidValue;
   if (a.out_split.hi && (!a.out_split.lo || !a.out_split.inv || a.out_split.chunk != kSplitChunkFine ||
                          a.d % kSplitChunkFine != 0))
     return hipErrorInvalidValue;
   if (kv == kKvF16 && prefill_attention_many_rows(a)) return launch_prefill_attention_many_rows(a, stream);
-  return kv == kKvF16 ? launch_prefill_attention_kv<__half>(a, stream)
-                      : launch_prefill_attention_kv<float>(a, stream);
+  if (a.pool.k)
+    return kv == kKvF16 ? launch_prefill_attention_kv<__half, true>(a, stream)
+                        : launch_prefill_attention_kv<float, true>(a, stream);
+  return kv == kKvF16 ? launch_prefill_attention_kv<__half, false>(a, stream)
+                      : launch_prefill_attention_kv<float, false>(a, stream);
 }
 
 }  // namespace mmr

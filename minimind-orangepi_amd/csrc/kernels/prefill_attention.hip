@@ -95,7 +95,7 @@ __device__ __forceinline__ void split8(const float* x, f16x8& hi, f16x8& lo) {
 // reads), which is what that kernel waits for on long prompts.  8 query heads
 // on 2, 3,000 rows from position 1,111: d 96 142.7 -> 72.6 us, d 64 95.4 ->
 // 56.2, d 32 69.6 -> 40.9; 4,096 rows from 0, d 96: 163.8 -> 78.3 us.
-template <int D>
+template <int D, bool kPool>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attention_f16_kernel(
     PrefillAttnArgs a) {
   constexpr int HB = kHeads, S = kWaves / HB;
@@ -125,6 +125,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const int qi = lane % 32, half = lane / 32;
   const int qpos = a.start + q0 + qi;
 
+  const int b = blockIdx.z;
   const int last_key = a.start + min(q0 + kQueryTile, a.tokens) - 1;
   const int n_tiles = last_key / kKeyTile + 1;
   const int n_iter = (n_tiles + S - 1) / S;
@@ -144,6 +145,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   };
   auto locate = [&](int i) {
     const int t0 = min(s + i * S, n_tiles - 1) * kKeyTile;
+    if constexpr (kPool) {
+      const int64_t off = kv_pool_offset(a.pool.interleave, b, t0, g, a.hkv, D) * 2;
+      return Tile{static_cast<const char*>(a.pool.k) + off, static_cast<const char*>(a.pool.v) + off, last_key - t0};
+    }
     const int seg = kv_segment(t0);
     const int64_t off = kv_segment_offset(seg, t0, g, a.hkv, D) * 2;
     return Tile{static_cast<const char*>(a.seg.s[seg].k) + off, static_cast<const char*>(a.seg.s[seg].v) + off,
@@ -182,7 +187,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   f16x8 qh[DJ], ql[DJ];
   {
     const float qscale = 1.4426950408889634f / sqrtf(static_cast<float>(D));
-    const float* qsrc = a.query + static_cast<int64_t>(min(q0 + qi, a.tokens - 1)) * a.query_stride + h * D + 8 * half;
+    const int64_t qrow = static_cast<int64_t>(b) * a.tokens + min(q0 + qi, a.tokens - 1);
+    const float* qsrc = a.query + qrow * a.query_stride + h * D + 8 * half;
 #pragma unroll
     for (int j = 0; j < DJ; ++j) {
       const float4 x0 = *reinterpret_cast<const float4*>(qsrc + 16 * j);
@@ -368,7 +374,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   if (s > 0) return;
   const float inv = 1.0f / half_swap_sum(l_part);
   const bool live = q0 + qi < a.tokens;
-  const int64_t row = static_cast<int64_t>(q0 + qi) * a.out_stride + h * D + 4 * half;
+  const int64_t orow = static_cast<int64_t>(b) * a.tokens + q0 + qi;
+  const int64_t row = orow * a.out_stride + h * D + 4 * half;
 #pragma unroll
   for (int j = 0; j < DT; ++j) {
     ot[j] *= inv;
@@ -401,7 +408,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
           *reinterpret_cast<f16x4*>(a.out_split.lo + row + 32 * j + 8 * q) = lo;
         }
         if (half == 0)
-          a.out_split.inv[static_cast<int64_t>(q0 + qi) * (a.hq * D / kSplitChunkFine) + h * DT + j] = ldexpf(1.0f, e - 15);
+          a.out_split.inv[orow * (a.hq * D / kSplitChunkFine) + h * DT + j] = ldexpf(1.0f, e - 15);
       }
     }
   }
@@ -422,16 +429,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 bool prefill_attention_many_rows(const PrefillAttnArgs& a) {
   if (a.d != 32 && a.d != 64 && a.d != 96) return false;
   if (a.hkv <= 0 || a.hq % a.hkv != 0 || a.hq / a.hkv % kHeads != 0) return false;
-  const int64_t blocks = int64_t{(a.tokens + kQueryTile - 1) / kQueryTile} * (a.hq / kHeads);
+  const int64_t blocks = int64_t{(a.tokens + kQueryTile - 1) / kQueryTile} * (a.hq / kHeads) * a.seqs;
   return blocks >= 112 || (blocks >= 80 && a.start >= a.tokens);
 }
 
+namespace {
+template <int D>
+void launch_many_rows(const PrefillAttnArgs& a, hipStream_t stream) {
+  const dim3 grid((a.tokens + kQueryTile - 1) / kQueryTile, a.hq / kHeads, a.seqs);
+  // The page lookup is a compile-time choice: a branch there would cut the
+  // step's matrix products into two blocks (82 -> 93 us a pass, 3,000 rows).
+  if (a.pool.k) {
+    prefill_attention_f16_kernel<D, true><<<grid, kThreads, 0, stream>>>(a);
+  } else {
+    prefill_attention_f16_kernel<D, false><<<grid, kThreads, 0, stream>>>(a);
+  }
+}
+}  // namespace
+
 hipError_t launch_prefill_attention_many_rows(const PrefillAttnArgs& a, hipStream_t stream) {
-  const dim3 grid((a.tokens + kQueryTile - 1) / kQueryTile, a.hq / kHeads);
   switch (a.d) {
-    case 32: prefill_attention_f16_kernel<32><<<grid, kThreads, 0, stream>>>(a); break;
-    case 64: prefill_attention_f16_kernel<64><<<grid, kThreads, 0, stream>>>(a); break;
-    case 96: prefill_attention_f16_kernel<96><<<grid, kThreads, 0, stream>>>(a); break;
+    case 32: launch_many_rows<32>(a, stream); break;
+    case 64: launch_many_rows<64>(a, stream); break;
+    case 96: launch_many_rows<96>(a, stream); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

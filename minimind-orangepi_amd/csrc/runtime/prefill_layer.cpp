@@ -100,6 +100,7 @@ void enqueue_prefill_layer(const MiniMindConfig& c, const LayerDev& w, const flo
   const int Hq = static_cast<int>(c.num_attention_heads), Hkv = static_cast<int>(c.num_key_value_heads);
   const int F = static_cast<int>(c.intermediate_size);
   const int qkv_w = (Hq + 2 * Hkv) * D;
+  if (kv.seqs < 1 || rows % kv.seqs != 0) throw std::invalid_argument("prefill rows do not divide into the sequences");
   const SplitChoice sc = split_choice(c, rows);
   float* const xf = sc.x ? nullptr : s.x;  // fp32 normalised rows, when the GEMMs read those
   const mmr::SplitPlanes* xs = sc.x ? &s.xs : nullptr;
@@ -160,7 +161,9 @@ void enqueue_prefill_layer(const MiniMindConfig& c, const LayerDev& w, const flo
   q.inv_freq = inv_freq;
   q.start = kv.rope_start;
   q.row0 = kv.row0;
-  q.tokens = rows;
+  q.tokens = rows / kv.seqs;
+  q.seqs = kv.seqs;
+  q.pool = kv.pool;
   q.seg = kv.seg;
   q.hq = Hq;
   q.hkv = Hkv;
@@ -168,12 +171,15 @@ void enqueue_prefill_layer(const MiniMindConfig& c, const LayerDev& w, const flo
   q.query = s.q;
   q.query_stride = Hq * D;
   check_hip(mmr::launch_qkv_rows(q, kv.dtype, stream), "prefill qkv rows");
+  if (!next_norm) return;
   mmr::PrefillAttnArgs at;
   at.query = s.q;
   at.query_stride = Hq * D;
   at.seg = kv.seg;
   at.start = kv.row0;
-  at.tokens = rows;
+  at.tokens = rows / kv.seqs;
+  at.seqs = kv.seqs;
+  at.pool = kv.pool;
   at.hq = Hq;
   at.hkv = Hkv;
   at.d = D;

@@ -51,6 +51,10 @@ struct PrefillKv {
   mmr::KvDtype dtype = mmr::kKvF32;
   int rope_start = 0;              // RoPE position of row 0
   int row0 = 0;                    // cache row of row 0 (rows 0 .. row0 - 1 already cached)
+  // A batch: the rows are `seqs` sequences' rows / seqs tokens each, one
+  // sequence after the other, all at the same positions; their cache is the pool.
+  int seqs = 1;
+  mmr::KvPool pool;
 };
 
 // One layer over rows 0 .. rows - 1.  On entry the scratch holds the rows of
@@ -58,7 +62,9 @@ struct PrefillKv {
 // the previous layer's call); h is the residual stream, updated in place.
 // Row i's query attends cache rows 0 .. row0 + i.  On exit the scratch holds
 // the new h normalised with `next_norm` (the next layer's input norm, or the
-// final norm with final_norm set).
+// final norm with final_norm set).  next_norm = nullptr: only the keys and
+// values are wanted (the last layer of a prompt whose rows predict nothing);
+// h and the scratch's rows are then undefined.
 void enqueue_prefill_layer(const MiniMindConfig& c, const LayerDev& w, const float* inv_freq, const PrefillScratch& s,
                            const PrefillKv& kv, int rows, float* h, const float* next_norm, bool final_norm,
                            hipStream_t stream);

@@ -127,6 +127,38 @@ def test_batch_sizes_across_gemm_paths(gpu, batch):
         assert rel_err(bs.read_logits(b), ref_logits) < 1e-4, b
 
 
+@pytest.mark.parametrize("batch,low,high,kv", [(2, 5, 5, "f32"), (2, 700, 720, "f16"), (33, 126, 150, "f16"),
+                                               (300, 30, 33, "f32")])
+def test_batch_prompt_rows_match_tokenwise(gpu, monkeypatch, batch, low, high, kv):
+    # the prompts through the prefill layers against the same prompts through
+    # the steps (MMR_PREFILL_TOKENWISE): the fewest rows that take them (4);
+    # 699 rows of two sequences (the many-rows attention over pages); 33 and
+    # 300 sequences, whose rows run in two and three passes (4,096 rows over
+    # the batch a pass), the last of them ragged
+    mmr = gpu
+    print(f"[case] batch prompt rows B={batch} {low}..{high} kv={kv}", flush=True)
+    g = load_golden("mini")
+    m = synth_model(mmr, g)
+    kvd = mmr.KV_F16 if kv == "f16" else mmr.KV_F32
+    rng = np.random.default_rng(batch + low)
+    lengths = [low] + [int(n) for n in rng.integers(low, high + 1, batch - 1)]
+    prompts = [[int(t) for t in rng.integers(0, g["config"]["vocab_size"], n)] for n in lengths]
+    steps = 6
+    last = max(lengths) + steps
+    monkeypatch.setenv("MMR_PREFILL_TOKENWISE", "1")
+    tok = m.make_batch_state(batch, last, kvd)
+    monkeypatch.delenv("MMR_PREFILL_TOKENWISE")
+    rows = m.make_batch_state(batch, last, kvd)
+    for st in (tok, rows):
+        st.prefill(prompts)
+        assert st.steps == max(lengths)
+        st.decode(steps)
+        st.synchronize()
+    for b in sorted({0, 1, batch // 2, batch - 1}):
+        np.testing.assert_array_equal(rows.read_sequence(b, 0, last + 1), tok.read_sequence(b, 0, last + 1))
+        assert rel_err(rows.read_logits(b), tok.read_logits(b)) < 1e-4, b
+
+
 def test_batch_reproduces_reference_golden(gpu):
     # MiniMind2 (configs[3] weights): sequence 0 holds the cfg3_short prompt,
     # whose greedy continuation is the reference CPU path's golden output
