@@ -1,0 +1,387 @@
+// gemm_rows.hip -- the prompt projection for many rows: C[m][n] = sum_k
+// A[m][k] * W[n][k] on 128 x 256 tiles of gfx950's fp16 matrix cores
+// (device_matmul / device_matmul_add with batch = seq_len, ascend_matmul.h:
+// 102-107).  prefill.hip has the kernels for fewer rows and other K, and the
+// rule that chooses.
+#include "device_common.h"
+#include "kernels.h"
+
+#include <type_traits>
+
+namespace mmr {
+namespace {
+
+using f32x16 = float __attribute__((ext_vector_type(16)));
+using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
+using f16x4 = _Float16 __attribute__((ext_vector_type(4)));
+
+constexpr int kBM = 128, kBN = 256, kBK = 64;
+constexpr int kWaves = 8, kThreads = kWaves * kWave;
+constexpr int kStages = 2;
+constexpr int kRowChunks = kBK / 8;
+constexpr int kPlaneBytes = kBM * kBK * 2;                     // one fp16 plane of A, one stage
+constexpr int kStageBytes = 2 * kPlaneBytes + kBN * kBK * 2;   // A hi, A lo, W
+constexpr int kActLd = kBN / 2 + 4;                            // floats per row of the act tile
+static_assert(kBM * kActLd * 4 <= kStages * kStageBytes, "act tile exceeds the stages");
+
+enum : int { kA32, kAPlanes };  // fp32 rows; fp16 planes with one scale per row
+enum : int { kStore, kResidual, kSwiGlu };
+
+// 16-byte chunk position of (row, chunk) in a stage [rows][8 chunks]: the 16
+// rows that a fragment read takes at one chunk lie in 16 distinct 16-byte
+// bank groups.
+__device__ __forceinline__ int chunk_pos(int row, int chunk) { return row * kRowChunks + (chunk ^ ((row >> 1) & 7)); }
+
+// Block = 128 x 256 of C, 8 waves of 64 x 64 (2 x 2 fragments of 32 x 32), K
+// in stages of 64: W and pre-split A by direct loads (whole 128-byte lines),
+// fp32 A through registers, where it is split hi + lo.  Per k step of 16 the
+// products are v_mfma_f32_32x32x16_f16 of the hi and the lo plane.
+//
+// What bounds it: LDS (a stage is 64 KB written and 192 KB read for 2,048
+// cycles of matrix products per SIMD) and, on real data, the clock, which the
+// products pull down (the same launch on degenerate data ran 10% faster).  The
+// 64 x 64 tiles of prefill.hip bring twice the bytes per product into LDS, and
+// read twice as many from it.  2,048 rows of fp32 A, W 4096 x 768: 57.7 ->
+// 36.2 us (447 -> 712 TFLOP/s of products); 4,096 rows 106 -> 67 us; pre-split
+// A, 6,000 rows: gate_up + SwiGLU 109 -> 85 us, QKV 39 -> 29 us.  (128 x 128
+// tiles of 4 waves, two blocks per CU: 101 and 36 us; 64 x 128 per wave with
+// one level of sums: 96 us and twice the error.)
+template <int kA, int kEpi>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_kernel(GemmArgs g) {
+  __shared__ __align__(16) char lds[kStages * kStageBytes];
+  // fp32 A: the factor by which stage b's rows' sums change scale; at the end
+  // (and for planes) the rows' 1 / s.
+  __shared__ __align__(16) float scale[kStages][kBM];
+
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave / 4, wn = wave % 4;
+  // Block id i runs on XCD i % 8: each XCD takes a contiguous run of tiles,
+  // ordered so that a run covers squares of up to 8 x 8 tiles, whose A rows and
+  // W rows its L2 holds.
+  const int mt = (g.m + kBM - 1) / kBM, nt = (g.n + kBN - 1) / kBN;
+  const int tiles = mt * nt, per_xcd = (tiles + kXcds - 1) / kXcds;
+  const int tile = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
+  if (tile >= tiles || static_cast<int>(blockIdx.x / kXcds) >= per_xcd) return;  // block-uniform
+  const int band = tile / (8 * nt), in_band = tile % (8 * nt);
+  const int band_rows = min(8, mt - band * 8);
+  const int m0 = (band * 8 + in_band % band_rows) * kBM, n0 = in_band / band_rows * kBN;
+  const int nk = g.k / kBK;  // even
+
+  // Direct loads: wave-wide load i fills rows 8 i .. + 7 of a plane (128 bytes
+  // each: whole cache lines); this wave takes loads wave, wave + 8, ...
+  constexpr int kALoads = kBM / 8 / kWaves, kWLoads = kBN / 8 / kWaves;
+  auto source = [&](int j, int r0, int rows, int64_t stride) {
+    const int row = (wave + kWaves * j) * 8 + lane / 8;
+    return static_cast<uint32_t>((min(r0 + row, rows - 1) * stride + ((lane % 8) ^ ((row >> 1) & 7)) * 8) * 2);
+  };
+  uint32_t a_off[kALoads], w_off[kWLoads];
+#pragma unroll
+  for (int j = 0; j < kALoads; ++j) a_off[j] = kA == kA32 ? 0 : source(j, m0, g.m, g.lda);
+#pragma unroll
+  for (int j = 0; j < kWLoads; ++j) w_off[j] = source(j, n0, g.n, g.k);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
+  auto issue = [&](int t, int buf) {
+    const int64_t kb = static_cast<int64_t>(t) * kBK * 2;
+    const uint32_t dst = lds0 + buf * kStageBytes + wave * 1024;
+    if constexpr (kA != kA32) {
+#pragma unroll
+      for (int j = 0; j < kALoads; ++j) {
+        dma_load<16>(reinterpret_cast<const char*>(g.a_hi) + kb, a_off[j], dst + j * kWaves * 1024);
+        dma_load<16>(reinterpret_cast<const char*>(g.a_lo) + kb, a_off[j], dst + j * kWaves * 1024 + kPlaneBytes);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kWLoads; ++j)
+      dma_load<16>(reinterpret_cast<const char*>(g.w) + kb, w_off[j], dst + j * kWaves * 1024 + 2 * kPlaneBytes);
+  };
+
+  // fp32 A: this thread's four 4-column pieces of a stage, row (tid + 512 u)
+  // / 16, columns 4 (tid % 16).  The 16 lanes of a row find its maximum
+  // together; the row's scale s = 2^(15 - e) follows the largest |a| seen so
+  // far, and the sums so far follow the scale (a power of two, exact).
+  constexpr int kPieces = kBM * kBK / 4 / kThreads;
+  float4 areg[kA == kA32 ? kPieces : 1];
+  int e_run[kA == kA32 ? kPieces : 1];
+  auto load_a = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) {
+      const int row = min(m0 + (tid + u * kThreads) / 16, g.m - 1);
+      areg[u] = *reinterpret_cast<const float4*>(g.a + static_cast<int64_t>(row) * g.lda + t * kBK + tid % 16 * 4);
+    }
+  };
+  auto store_a = [&](int buf, int u0, int u1) {
+#pragma unroll
+    for (int u = u0; u < u1; ++u) {
+      const int row = (tid + u * kThreads) / 16, q = tid % 16;
+      const float4 v = areg[u];
+      const float mx = group_max<16>(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+      const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx), e_run[u]) : e_run[u];
+      const float sc = ldexpf(1.0f, 15 - e);
+      const float x[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
+      f16x4 hi, lo;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        hi[j] = static_cast<_Float16>(x[j]);
+        lo[j] = static_cast<_Float16>(x[j] - static_cast<float>(hi[j]));
+      }
+      char* dst = lds + buf * kStageBytes + chunk_pos(row, q / 2) * 16 + q % 2 * 8;
+      *reinterpret_cast<f16x4*>(dst) = hi;
+      *reinterpret_cast<f16x4*>(dst + kPlaneBytes) = lo;
+      if (q == 0) scale[buf][row] = ldexpf(1.0f, e_run[u] - e);
+      e_run[u] = e;
+    }
+  };
+
+  const int half = lane / 32, l32 = lane % 32;
+  // Fragment addresses within a stage; the next 32 rows (columns) are 4 KB on.
+  int a_rd[4], w_rd[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    a_rd[ks] = chunk_pos(wm * 64 + l32, 2 * ks + half) * 16;
+    w_rd[ks] = chunk_pos(wn * 64 + l32, 2 * ks + half) * 16 + 2 * kPlaneBytes;
+  }
+  f32x16 acc[2][2], part[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+  struct Frags {
+    f16x8 ah[2], al[2], w[2];
+  };
+  auto read = [&](Frags& f, int buf, int ks) {
+    const char* st = lds + buf * kStageBytes;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f.ah[i] = *reinterpret_cast<const f16x8*>(st + a_rd[ks] + i * 4096);
+      f.al[i] = *reinterpret_cast<const f16x8*>(st + a_rd[ks] + i * 4096 + kPlaneBytes);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) f.w[j] = *reinterpret_cast<const f16x8*>(st + w_rd[ks] + j * 4096);
+  };
+  // Sums run in two levels: the products of kSplitChunk columns (one stage of
+  // fp32 A) in `part`, then into `acc`; a single chain of K / 16 additions
+  // doubled the error against 64 bits.
+  auto multiply = [&](const Frags& f, bool fresh) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.w[j], fresh ? f32x16{} : part[i][j], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.w[j], part[i][j], 0, 0, 0);
+  };
+  auto flush = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
+  };
+  // The sums of the rows times their factors.
+  auto rescale = [&](const float* factors) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 sv = *reinterpret_cast<const float4*>(factors + wm * 64 + i * 32 + 8 * q + 4 * half);
+        const float s4[4] = {sv.x, sv.y, sv.z, sv.w};
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] *= s4[r];
+      }
+  };
+
+  // Each k step's fragments are read while the one before is multiplied,
+  // across stages too.  Stage t + 1 has to be in LDS, and stage t's last
+  // fragments in registers, before stage t's last products; then stage t's
+  // buffer takes stage t + 2.
+  {
+    issue(0, 0);
+    if constexpr (kA == kA32) {
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) e_run[u] = -100;
+      load_a(0);
+      store_a(0, 0, kPieces);
+    }
+    issue(1, 1);
+    if constexpr (kA == kA32) load_a(1);
+    // Stage 0 has landed (fp32 A: its W, waited for with A).
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                 :
+                 : "n"((kA == kA32 ? kPieces : 2 * kALoads) + kWLoads)
+                 : "memory");
+    Frags f0, f1;
+    read(f0, 0, 0);
+    float factor = 1.0f;
+    auto step = [&](int t, int buf, bool fresh, bool last) {
+      if constexpr (kA == kA32) {
+        if (__any(factor != 1.0f)) rescale(&scale[buf][0]);
+      }
+      read(f1, buf, 1);
+      multiply(f0, fresh);
+      if constexpr (kA == kA32) {
+        if (t + 1 < nk) store_a(buf ^ 1, 0, kPieces / 2);
+      }
+      read(f0, buf, 2);
+      multiply(f1, false);
+      if constexpr (kA == kA32) {
+        if (t + 1 < nk) store_a(buf ^ 1, kPieces / 2, kPieces);
+      }
+      read(f1, buf, 3);
+      multiply(f0, false);
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (t + 2 < nk) {
+        issue(t + 2, buf);
+        if constexpr (kA == kA32) load_a(t + 2);
+      }
+      if constexpr (kA == kA32) factor = scale[buf ^ 1][wm * 64 + lane];
+      read(f0, buf ^ 1, 0);  // past the last stage: stale, not used
+      multiply(f1, false);
+      if (last) flush();
+    };
+    for (int t = 0; t < nk; t += 2) {
+      step(t, 0, true, kA == kA32);
+      step(t + 1, 1, kA == kA32, true);
+    }
+  }
+  // The rows' 1 / s.
+  __syncthreads();
+  if constexpr (kA == kA32) {
+    if (tid % 16 == 0) {
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) scale[0][(tid + u * kThreads) / 16] = ldexpf(1.0f, e_run[u] - 15);
+    }
+  } else if (tid < kBM) {
+    scale[0][tid] = g.a_inv[static_cast<int64_t>(min(m0 + tid, g.m - 1)) * (g.k / kSplitChunk)];
+  }
+  __syncthreads();
+  rescale(&scale[0][0]);
+
+  // Lane: column l32 of each 32 x 32 fragment, rows 8 q + 4 half + r.
+  if constexpr (kEpi == kSwiGlu) {
+    // Gate column 2c in lane 2c, up column in lane 2c + 1: after one exchange
+    // the even lane forms act for rows r = 0, 1 and the odd lane for 2, 3;
+    // act goes through LDS so that a thread writes 4 columns of a row.
+    __syncthreads();
+    float* act = reinterpret_cast<float*>(lds);
+    const bool odd = (lane & 1) != 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float v[4], x[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            v[r] = acc[i][j][4 * q + r];
+            x[r] = dpp_move<dpp::kQuadXor1>(v[r]);
+          }
+          const float gate[2] = {odd ? x[2] : v[0], odd ? x[3] : v[1]};
+          const float up[2] = {odd ? v[2] : x[0], odd ? v[3] : x[1]};
+          const int row = wm * 64 + i * 32 + 8 * q + 4 * half + (odd ? 2 : 0), col = (wn * 64 + j * 32 + l32) / 2;
+#pragma unroll
+          for (int r = 0; r < 2; ++r) act[(row + r) * kActLd + col] = silu_fast(gate[r]) * up[r];
+        }
+    __syncthreads();
+    const int nkc = g.n / 2 / kSplitChunkFine;
+#pragma unroll
+    for (int p = 0; p < kBM * kBN / 8 / kThreads; ++p) {
+      const int idx = tid + p * kThreads, r = idx / (kBN / 8), c4 = idx % (kBN / 8);
+      const int row = m0 + r, col = n0 / 2 + c4 * 4;
+      const bool ok = row < g.m && col < g.n / 2;
+      const float4 v = *reinterpret_cast<const float4*>(&act[r * kActLd + c4 * 4]);
+      const int64_t off = static_cast<int64_t>(row) * g.ldc + col;
+      if (!g.act_split.hi) {
+        if (ok) *reinterpret_cast<float4*>(g.c + off) = v;
+        continue;
+      }
+      const float top = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+      const float mx = group_max<kSplitChunkFine / 4>(ok ? top : 0.0f);
+      int e = 0;
+      frexpf(mx, &e);  // e = 0 for a zero chunk
+      e = max(e, -100);
+      const float sc = ldexpf(1.0f, 15 - e);
+      const float x[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
+      f16x4 hi, lo;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        hi[j] = static_cast<_Float16>(x[j]);
+        lo[j] = static_cast<_Float16>(x[j] - static_cast<float>(hi[j]));
+      }
+      if (ok) {
+        *reinterpret_cast<f16x4*>(g.act_split.hi + off) = hi;
+        *reinterpret_cast<f16x4*>(g.act_split.lo + off) = lo;
+        if (c4 % (kSplitChunkFine / 4) == 0)
+          g.act_split.inv[static_cast<int64_t>(row) * nkc + col / kSplitChunkFine] = ldexpf(1.0f, e - 15);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int col = n0 + wn * 64 + j * 32 + l32;
+        const int base = m0 + wm * 64 + i * 32 + 4 * half;
+        float res[16];
+        if constexpr (kEpi == kResidual) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            res[e] = g.residual[static_cast<int64_t>(min(base + 8 * (e / 4) + e % 4, g.m - 1)) * g.ldc + min(col, g.n - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int row = base + 8 * (e / 4) + e % 4;
+          if (row < g.m && col < g.n)
+            g.c[static_cast<int64_t>(row) * g.ldc + col] = kEpi == kResidual ? res[e] + acc[i][j][e] : acc[i][j][e];
+        }
+      }
+  }
+}
+
+template <int kA>
+void launch(const GemmArgs& g, hipStream_t s) {
+  const int tiles = ((g.m + kBM - 1) / kBM) * ((g.n + kBN - 1) / kBN);
+  const int grid = (tiles + kXcds - 1) / kXcds * kXcds;
+  if (g.swiglu) {
+    gemm_rows_kernel<kA, kSwiGlu><<<grid, kThreads, 0, s>>>(g);
+  } else if (g.residual) {
+    gemm_rows_kernel<kA, kResidual><<<grid, kThreads, 0, s>>>(g);
+  } else {
+    gemm_rows_kernel<kA, kStore><<<grid, kThreads, 0, s>>>(g);
+  }
+}
+
+}  // namespace
+
+// Tiles of this kernel enough for it, against prefill.hip's smaller ones: a
+// block takes a CU to itself, so a launch takes as long as one block per
+// round of 256, and from 96 tiles on that is the shorter (fp32 A, prefill.hip
+// / this one: 88 tiles, 1,000 rows of 2816 x 512, 24.4 / 22.3 us; 96 tiles,
+// 4,096 rows of 768 x 2048, 77.0 / 72.2; 80 tiles, 2,048 rows of 1152 x 768,
+// 32.1 / 30.3; 64 tiles, 4,096 rows of 512 x 1408, 46.2 / 51.9; 128 tiles,
+// 1,000 rows of 4096 x 768, 33.3 / 33.3; 352 tiles, 4,096 rows of 2816 x 512,
+// 59.9 / 44.8).
+bool gemm_many_rows(const GemmArgs& g) {
+  const int64_t a_bytes = static_cast<int64_t>(g.m) * g.lda * 2, w_bytes = static_cast<int64_t>(g.n) * g.k * 2;
+  const int64_t tiles = static_cast<int64_t>((g.m + kBM - 1) / kBM) * ((g.n + kBN - 1) / kBN);
+  return tiles >= 96 && tiles < (1 << 30) && g.k_splits == 1 && !g.register_staged && g.k % (2 * kBK) == 0 &&
+         (!g.a_hi || g.a_chunk == kSplitChunk) && (!g.swiglu || (g.n % 8 == 0 && g.ldc % 4 == 0)) &&
+         (reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.a_hi) | reinterpret_cast<uintptr_t>(g.a_lo) |
+          reinterpret_cast<uintptr_t>(g.w)) % 16 == 0 &&
+         a_bytes < (int64_t{1} << 32) && w_bytes < (int64_t{1} << 32);
+}
+
+hipError_t launch_gemm_many_rows(const GemmArgs& g, hipStream_t stream) {
+  if (g.a_hi) {
+    launch<kAPlanes>(g, stream);
+  } else {
+    launch<kA32>(g, stream);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace mmr

@@ -282,7 +282,9 @@ hipError_t launch_qkv_postprocess(const QkvPostArgs& a, KvDtype kv, hipStream_t 
 // `chunk`-wide column chunk a power-of-two scale s (the chunk's max |a|
 // mapped into [2^14, 2^15)), hi = fp16(s a), lo = fp16(s a - hi), inv = 1 / s.
 // Written once by the kernel producing A, staged by every GEMM block.
-// kSplitChunk (one scale per GEMM K tile) is staged as is; kSplitChunkFine
+// kSplitChunk (one scale per GEMM K tile) is staged as is; its writer, the
+// residual + norm kernel, sees whole rows and gives every chunk of a row the
+// same scale, which the many-rows GEMM relies on.  kSplitChunkFine
 // suits producers that see 32 columns at a time (attention heads, the SwiGLU
 // epilogue) and is brought to one scale per K tile while staging.
 constexpr int kSplitChunk = 128;
@@ -339,6 +341,10 @@ bool gemm_presplit_supported(int m, int n, int k);
 // n a multiple of 64.
 bool gemm_swiglu_split_supported(int m, int n, int k);
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
+// The kernel for many rows (gemm_rows.hip), which launch_gemm takes where it
+// is the faster one.
+bool gemm_many_rows(const GemmArgs& g);
+hipError_t launch_gemm_many_rows(const GemmArgs& g, hipStream_t stream);
 
 // A batch's KV page pools ([page][Hkv][kKvPage][D], see AttnArgs): page p of
 // sequence b is physical page p * interleave + b.  k = nullptr: none.

@@ -1273,6 +1273,7 @@ hipError_t launch_gemm(const GemmArgs& g, hipStream_t s) {
   if (g.k_splits < 1 || (g.k_splits > 1 && (g.residual || g.split_stride < static_cast<int64_t>(g.m) * g.ldc ||
                                             g.k_splits > gemm_k_splits(g.m, g.n, g.k))))
     return hipErrorInvalidValue;
+  if (gemm_many_rows(g)) return launch_gemm_many_rows(g, s);
   // Few rows (batched decode): stream W with one block per 16 rows of W.
   if (use_skinny(g.m, g.k)) return g.m <= 16 ? launch_gemm_skinny<1>(g, s) : launch_gemm_skinny<2>(g, s);
   // Calls with the chooser's split count take its tile.

@@ -428,6 +428,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // the registers of two waves per SIMD.)
 bool prefill_attention_many_rows(const PrefillAttnArgs& a) {
   if (a.d != 32 && a.d != 64 && a.d != 96) return false;
+  if ((reinterpret_cast<uintptr_t>(a.query) | reinterpret_cast<uintptr_t>(a.out)) % 16 != 0 ||
+      (a.query_stride | a.out_stride) % 4 != 0)
+    return false;  // rows are read and written 16 bytes at a time
   if (a.hkv <= 0 || a.hq % a.hkv != 0 || a.hq / a.hkv % kHeads != 0) return false;
   const int64_t blocks = int64_t{(a.tokens + kQueryTile - 1) / kQueryTile} * (a.hq / kHeads) * a.seqs;
   return blocks >= 112 || (blocks >= 80 && a.start >= a.tokens);

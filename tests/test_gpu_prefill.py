@@ -51,6 +51,38 @@ def test_matmul_matches_fp64_and_oracle(gpu, oracle, batch, rows, cols):
     assert rel_err(dr.numpy(), res + exact) < 1e-5
 
 
+@pytest.mark.parametrize("batch,rows,cols,grow", [(1409, 1793, 128, 0), (1536, 2048, 256, 0), (1500, 1800, 1408, 0),
+                                                  (1409, 2047, 768, 1), (1409, 2047, 768, -1)])
+def test_matmul_many_rows_matches_fp64(gpu, batch, rows, cols, grow):
+    # the 128 x 256 tiles (96 of them): a last row tile of 1 row, a last column
+    # tile of 1 column, the shortest K, an odd number of 128-column chunks;
+    # rows whose values grow or shrink by 2^60 along K (the running row scale),
+    # every row by another offset.  Against 64 bits, each row over its own
+    # scale: the planes hold 22 bits of the row's largest values (2.4e-7), the
+    # sums are fp32 over at most 1,408 products of like size (40 ulp at most).
+    mmr = gpu
+    print(f"[case] matmul many rows {batch}x{rows}x{cols} grow={grow}", flush=True)
+    rng = np.random.default_rng(batch + rows + cols)
+    w16, w32 = f16_weights(rng, rows, cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    if grow:
+        x *= np.exp2(np.linspace(-30, 30, cols) * grow + rng.integers(-9, 9, (batch, 1))).astype(np.float32)
+    x[7] = 0.0
+    dw, dx = mmr.DeviceArray.from_numpy(w16.view(np.uint16)), mmr.DeviceArray.from_numpy(x)
+    dy = mmr.DeviceArray((batch, rows), np.float32)
+    mmr.matmul_f16(dw, rows, cols, dx, batch, dy)
+    got = dy.numpy().astype(np.float64)
+    exact = x.astype(np.float64) @ w32.astype(np.float64).T
+    scale = np.maximum(np.abs(exact).max(axis=1, keepdims=True), 1e-30)
+    assert np.max(np.abs(got - exact) / scale) < 1e-5
+    assert not got[7].any()
+    if not grow:
+        res = rng.standard_normal((batch, rows)).astype(np.float32)
+        dr = mmr.DeviceArray.from_numpy(res)
+        mmr.matmul_f16(dw, rows, cols, dx, batch, dr, residual=dr)
+        assert rel_err(dr.numpy(), res + exact) < 1e-5
+
+
 def test_matmul_rejects_bad_shapes(gpu):
     mmr = gpu
     d = mmr.DeviceArray(64, np.float32)
