@@ -80,6 +80,12 @@ struct DeviceState {
   int64_t pf_chunk = 0;
   float* pf_h = nullptr;    // [chunk][H] residual stream
   PrefillScratch pf;        // the layer's scratch for pf_chunk rows
+  // The same for longer prompts (up to pf_long rows a pass), allocated by the
+  // first prompt that needs it.
+  int64_t pf_long = 0;
+  DeviceBuffer pf_long_buf;
+  float* pf_long_h = nullptr;
+  PrefillScratch pf_long_scratch;
   bool prefill_tokenwise = false;  // prefill through the decode step instead of the GEMM path
   hipStream_t stream = nullptr;
   std::map<std::pair<int, int>, hipGraphExec_t> graphs;  // (attention splits, steps) -> captured steps
@@ -113,8 +119,14 @@ namespace {
 // against 144, same box).  The count never falls as the context grows
 // (decode_attention_splits).
 constexpr int kMaxSplits = 512;
-// Prompt tokens per prefill chunk (GEMM rows); longer prompts run in chunks.
+// Prompt tokens of one pass of the prefill layers (GEMM rows).  Prompts of up
+// to kPrefillChunk run in one pass on buffers that every state has; longer ones
+// in as few equal passes of up to kPrefillLongChunk rows as they need, whose
+// larger GEMMs and attention launches fill the GPU (6,000 tokens of MiniMind2,
+// fp16 cache: passes of 512 rows 15.3 ms, 2,048 8.4 ms, 6,000 7.1 ms, before
+// the many-rows GEMM), on buffers of about 40 KB a row.
 constexpr int64_t kPrefillChunk = 512;
+constexpr int64_t kPrefillLongChunk = 4096;
 
 void require_size(const std::vector<float>& v, int64_t expected, const std::string& name) {
   if (static_cast<int64_t>(v.size()) != expected) throw std::invalid_argument(name + " has invalid size");
@@ -329,7 +341,8 @@ DecoderState LanguageModel::make_state(int64_t capacity, KvCacheDtype kv) const 
   ar.plan(device_->plan_lm.blocks * 4);
   ar.plan(device_->plan_lm.blocks * 4);
   int64_t chunk = kPrefillChunk;
-  if (const char* pc = std::getenv("MMR_PREFILL_CHUNK")) chunk = std::max<int64_t>(1, std::atoll(pc));
+  s->pf_long = kPrefillLongChunk;
+  if (const char* pc = std::getenv("MMR_PREFILL_CHUNK")) s->pf_long = chunk = std::max<int64_t>(1, std::atoll(pc));
   s->pf_chunk = s->prefill_tokenwise ? 0 : std::min<int64_t>(capacity, chunk);
   const int64_t C = s->pf_chunk;
   const std::size_t pf_bytes = C > 0 ? prefill_scratch_bytes(c, C) : 0;
@@ -669,18 +682,20 @@ void enqueue_step_kernels(const DeviceState& s, int splits, bool first = true, b
 // decoder_layer.cpp:661-734, chunked): embedding rows -> per layer RMSNorm
 // rows, qkv GEMM, q/k norm + RoPE + KV write, causal attention, O GEMM +
 // residual, RMSNorm rows, gate_up GEMM, SwiGLU rows, down GEMM + residual.
-// The residual stream of the chunk ends in s.pf_h.
-void enqueue_prefill_chunk(const DeviceState& s, int64_t start, int64_t n) {
+// The residual stream of the chunk ends in h; unless `wanted`, the last layer
+// stops after its keys and values (nothing else of it is read later).
+void enqueue_prefill_chunk(const DeviceState& s, int64_t start, int64_t n, float* h, const PrefillScratch& scratch,
+                           bool wanted) {
   const DeviceModel& m = *s.model;
   const auto& c = m.cfg;
   const int rows = static_cast<int>(n);
   check_hip(mmr::launch_embedding_gather(m.embed, s.seq + start, rows, static_cast<int>(c.vocab_size),
-                                         static_cast<int>(c.hidden_size), s.pf_h, s.err, s.stream),
+                                         static_cast<int>(c.hidden_size), h, s.err, s.stream),
             "prefill embedding");
   // Layer 0's input norm; every later layer's comes from the previous
   // layer's residual consumer (after the last layer the final norm, whose
   // rows are not used: the head normalises the last row itself).
-  enqueue_prefill_input_norm(c, s.pf, rows, s.pf_h, m.layers[0].input_norm, s.stream);
+  enqueue_prefill_input_norm(c, scratch, rows, h, m.layers[0].input_norm, s.stream);
   const size_t L = m.layers.size();
   for (size_t l = 0; l < L; ++l) {
     PrefillKv kv;
@@ -689,9 +704,21 @@ void enqueue_prefill_chunk(const DeviceState& s, int64_t start, int64_t n) {
     kv.rope_start = static_cast<int>(start);
     kv.row0 = static_cast<int>(start);
     const bool last = l + 1 == L;
-    enqueue_prefill_layer(c, m.layers[l], m.inv_freq, s.pf, kv, rows, s.pf_h,
-                          last ? m.final_norm : m.layers[l + 1].input_norm, last, s.stream);
+    enqueue_prefill_layer(c, m.layers[l], m.inv_freq, scratch, kv, rows, h,
+                          last ? (wanted ? m.final_norm : nullptr) : m.layers[l + 1].input_norm, last, s.stream);
   }
+}
+
+// Buffers of a prefill pass of `rows` rows (the stream is idle: nothing reads
+// the previous ones).
+void reserve_long_prefill(DeviceState& s, int64_t rows) {
+  const auto& c = s.model->cfg;
+  const std::size_t h_bytes = Arena::round_up(static_cast<std::size_t>(rows * c.hidden_size) * sizeof(float));
+  s.pf_long_scratch = PrefillScratch{};
+  s.pf_long_buf.reset(h_bytes + prefill_scratch_bytes(c, rows));
+  s.pf_long_h = static_cast<float*>(s.pf_long_buf.data());
+  s.pf_long_scratch = carve_prefill_scratch(c, rows, static_cast<char*>(s.pf_long_buf.data()) + h_bytes);
+  s.pf_long_scratch.register_staged = s.pf.register_staged;
 }
 
 // `steps` consecutive decode steps with one attention split count, as one
@@ -821,15 +848,24 @@ void LanguageModel::enqueue_prefill(DecoderState& state, const std::vector<int32
   // finalize kernel writes the prediction to seq[position + n] and advances
   // the position past the prompt, exactly as the last decode step would.
   const int64_t start = state.position;
-  int64_t last_rows = 0;
-  for (int64_t b = start; b < start + n; b += s.pf_chunk) {
-    last_rows = std::min<int64_t>(s.pf_chunk, start + n - b);
-    enqueue_prefill_chunk(s, b, last_rows);
+  int64_t last_rows = 0, chunk = s.pf_chunk;
+  float* h = s.pf_h;
+  const PrefillScratch* scratch = &s.pf;
+  if (n > chunk && s.pf_long > chunk) {
+    const int64_t passes = (n + s.pf_long - 1) / s.pf_long;
+    chunk = (n + passes - 1) / passes;
+    if (s.pf_long_scratch.rows < chunk) reserve_long_prefill(s, chunk);
+    h = s.pf_long_h;
+    scratch = &s.pf_long_scratch;
+  }
+  for (int64_t b = start; b < start + n; b += chunk) {
+    last_rows = std::min<int64_t>(chunk, start + n - b);
+    enqueue_prefill_chunk(s, b, last_rows, h, *scratch, b + last_rows == start + n);
   }
   s.staging[s.capacity + 2] = static_cast<int32_t>(start + n - 1);
   check_hip(hipMemcpyAsync(s.pos, s.staging + s.capacity + 2, sizeof(int32_t), hipMemcpyHostToDevice, s.stream),
             "hipMemcpyAsync pos");
-  check_hip(hipMemcpyAsync(s.h, s.pf_h + (last_rows - 1) * config_.hidden_size, config_.hidden_size * sizeof(float),
+  check_hip(hipMemcpyAsync(s.h, h + (last_rows - 1) * config_.hidden_size, config_.hidden_size * sizeof(float),
                            hipMemcpyDeviceToDevice, s.stream),
             "hipMemcpyAsync last row");
   const int splits = choose_splits(start + n, mmr::attention_tile_tokens(static_cast<int>(config_.head_dim)));

@@ -311,6 +311,28 @@ def test_minimind2_ragged_chunks_match_tokenwise(gpu, monkeypatch, prompt_len):
     assert gem.read_sequence(prompt_len, 1).tolist() == tok.read_sequence(prompt_len, 1).tolist()
 
 
+@pytest.mark.parametrize("prompt_len", [2500, 5000])
+def test_minimind2_long_passes_match_chunks(gpu, monkeypatch, prompt_len):
+    # one pass of 2,500 rows and two of them (the many-rows GEMM for QKV and
+    # gate_up, the many-rows attention after 2,500 cached rows) against the
+    # same prompt in 512-row chunks: same next token, logits within 1e-4 (fp16
+    # K/V roundings of differently grouped fp32 sums, as in the tests below)
+    mmr = gpu
+    print(f"[case] MiniMind2 long prefill rows={prompt_len}", flush=True)
+    g = load_golden("cfg3_short")
+    m = synth_model(mmr, g)
+    prompt = mmr.synthesize_prompt(12, prompt_len, 6400).tolist()
+    monkeypatch.setenv("MMR_PREFILL_CHUNK", "512")
+    chunks = m.make_state(prompt_len + 8, mmr.KV_F16)
+    monkeypatch.delenv("MMR_PREFILL_CHUNK")
+    passes = m.make_state(prompt_len + 8, mmr.KV_F16)
+    for st in (chunks, passes):
+        st.enqueue_prefill(prompt)
+        st.synchronize()
+    assert rel_err(passes.read_logits(), chunks.read_logits()) < 1e-4
+    assert passes.read_sequence(prompt_len, 1).tolist() == chunks.read_sequence(prompt_len, 1).tolist()
+
+
 def test_gemm_kernels_agree(gpu, monkeypatch):
     # the direct-to-LDS GEMM (pre-split A, K % 64 == 0) against the
     # register-staged one (MMR_GEMM_REGISTER_STAGED=1) on a MiniMind2 prefill
