@@ -409,10 +409,10 @@ struct PrefillAttnArgs {
   KvPool pool;
 };
 hipError_t launch_prefill_attention(const PrefillAttnArgs& a, KvDtype kv, hipStream_t stream);
-// The kernel for many rows of an fp16 cache (prefill_attention.hip), which
-// launch_prefill_attention takes where it is the faster one.
-bool prefill_attention_many_rows(const PrefillAttnArgs& a);
-hipError_t launch_prefill_attention_many_rows(const PrefillAttnArgs& a, hipStream_t stream);
+// The kernels for many rows (prefill_attention.hip), which
+// launch_prefill_attention takes where they are the faster ones.
+bool prefill_attention_many_rows(const PrefillAttnArgs& a, KvDtype kv);
+hipError_t launch_prefill_attention_many_rows(const PrefillAttnArgs& a, KvDtype kv, hipStream_t stream);
 
 // --------------------------------------------------------------- batch ----
 // Decode of a batch of independent sequences, sequence b at its own device

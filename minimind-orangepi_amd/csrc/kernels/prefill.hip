@@ -1313,7 +1313,7 @@ hipError_t launch_prefill_attention(const PrefillAttnArgs& a, KvDtype kv, hipStr
   if (a.out_split.hi && (!a.out_split.lo || !a.out_split.inv || a.out_split.chunk != kSplitChunkFine ||
                          a.d % kSplitChunkFine != 0))
     return hipErrorInvalidValue;
-  if (kv == kKvF16 && prefill_attention_many_rows(a)) return launch_prefill_attention_many_rows(a, stream);
+  if (prefill_attention_many_rows(a, kv)) return launch_prefill_attention_many_rows(a, kv, stream);
   if (a.pool.k)
     return kv == kKvF16 ? launch_prefill_attention_kv<__half, true>(a, stream)
                         : launch_prefill_attention_kv<float, true>(a, stream);

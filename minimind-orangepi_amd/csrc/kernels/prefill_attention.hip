@@ -1,9 +1,9 @@
-// prefill_attention.hip -- causal attention of many prompt rows over an fp16
-// KV cache on gfx950's matrix cores (the reference's device_prefill_attention,
+// prefill_attention.hip -- causal attention of many prompt rows on gfx950's
+// matrix cores (the reference's device_prefill_attention,
 // ascend_custom_ops.h:122-130; per token decoder_layer.cpp:184-234): `tokens`
 // queries at positions start .. start + tokens - 1 attend cache keys 0 ..
-// their own position.  prefill.hip has the kernel for fewer rows, an fp32
-// cache and the other head shapes, and the rule that chooses.
+// their own position.  One kernel for an fp16 cache and one for an fp32 one;
+// prefill.hip has the kernel for fewer rows and the other head shapes.
 #include "device_common.h"
 #include "kernels.h"
 
@@ -14,6 +14,7 @@ namespace {
 
 using f32x2 = float __attribute__((ext_vector_type(2)));
 using f16x2 = _Float16 __attribute__((ext_vector_type(2)));
+using f32x4 = float __attribute__((ext_vector_type(4)));
 using f32x16 = float __attribute__((ext_vector_type(16)));
 using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
 using f16x4 = _Float16 __attribute__((ext_vector_type(4)));
@@ -57,16 +58,114 @@ __device__ __forceinline__ float half_swap_sum(float v) {
 // x = hi + lo in fp16, each rounded to nearest: 22 significant bits.  lo =
 // fp16(x - hi) is one instruction per value: hi * -1 + x, exact in fp32,
 // converted by v_fma_mix as it is written.
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, f16x2));
+  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(x0));
+  asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(x1));
+}
 __device__ __forceinline__ void split8(const float* x, f16x8& hi, f16x8& lo) {
   uint32_t h[4], l[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x[2 * e], x[2 * e + 1]}, f16x2));
-    asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l[e]) : "v"(h[e]), "v"(x[2 * e]));
-    asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l[e]) : "v"(h[e]), "v"(x[2 * e + 1]));
-  }
+  for (int e = 0; e < 4; ++e) split2(x[2 * e], x[2 * e + 1], h[e], l[e]);
   hi = __builtin_bit_cast(f16x8, u32x4{h[0], h[1], h[2], h[3]});
   lo = __builtin_bit_cast(f16x8, u32x4{l[0], l[1], l[2], l[3]});
+}
+
+// Sum of a tile's 16 probabilities in a tree: added one by one to the running
+// sum, thousands of keys cost it several units in the last place.
+__device__ __forceinline__ float sum16(const float (&p)[16]) {
+  float s[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) s[q] = (p[4 * q] + p[4 * q + 1]) + (p[4 * q + 2] + p[4 * q + 3]);
+  return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+// The end of a block: the key ranges' (m, l) per query and O^T, as the lanes
+// of wave (s, hb) hold them, merge pairwise through `mrg`, and range 0's waves
+// write the rows.
+template <int D, int HB>
+__device__ __forceinline__ void merge_and_write(const PrefillAttnArgs& a, f32x16 (&ot)[D / 32], float m_run,
+                                                float l_part, float* mrg, int s, int hb, int lane, int h, int b,
+                                                int q0) {
+  constexpr int S = kWaves / HB, DT = D / 32;
+  constexpr int kMergeFloats = (D / 2 + 2) * kWave;
+  const int qi = lane % 32, half = lane / 32;
+#pragma unroll
+  for (int step = S / 2; step >= 1; step /= 2) {
+    __syncthreads();  // the stages (or the previous round's values) have been read
+    if (s >= step && s < 2 * step) {
+      float* dst = mrg + ((s - step) * HB + hb) * kMergeFloats;
+#pragma unroll
+      for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(dst + ((j * 4 + q) * kWave + lane) * 4) =
+              make_float4(ot[j][4 * q], ot[j][4 * q + 1], ot[j][4 * q + 2], ot[j][4 * q + 3]);
+      dst[D / 2 * kWave + lane] = m_run;
+      dst[D / 2 * kWave + kWave + lane] = l_part;
+    }
+    __syncthreads();
+    if (s < step) {
+      const float* src = mrg + (s * HB + hb) * kMergeFloats;
+      const float m_b = src[D / 2 * kWave + lane], l_b = src[D / 2 * kWave + kWave + lane];
+      const float m_new = fmaxf(m_run, m_b);
+      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+      const float ea = __builtin_amdgcn_exp2f(m_run - m_use), eb = __builtin_amdgcn_exp2f(m_b - m_use);
+      l_part = l_part * ea + l_b * eb;
+      m_run = m_new;
+#pragma unroll
+      for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4 v = *reinterpret_cast<const float4*>(src + ((j * 4 + q) * kWave + lane) * 4);
+          ot[j][4 * q] = fmaf(v.x, eb, ot[j][4 * q] * ea);
+          ot[j][4 * q + 1] = fmaf(v.y, eb, ot[j][4 * q + 1] * ea);
+          ot[j][4 * q + 2] = fmaf(v.z, eb, ot[j][4 * q + 2] * ea);
+          ot[j][4 * q + 3] = fmaf(v.w, eb, ot[j][4 * q + 3] * ea);
+        }
+    }
+  }
+  if (s > 0) return;
+  const float inv = 1.0f / half_swap_sum(l_part);
+  const bool live = q0 + qi < a.tokens;
+  const int64_t orow = static_cast<int64_t>(b) * a.tokens + q0 + qi;
+  const int64_t row = orow * a.out_stride + h * D + 4 * half;
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    ot[j] *= inv;
+    if (a.out && live) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<float4*>(a.out + row + 32 * j + 8 * q) =
+            make_float4(ot[j][4 * q], ot[j][4 * q + 1], ot[j][4 * q + 2], ot[j][4 * q + 3]);
+    }
+    if (a.out_split.hi) {  // the 32 dims of slice j are one chunk: 16 here, 16 in the other half
+      float mx = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(ot[j][i]));
+      mx = half_swap_max(mx);
+      int e = 0;
+      frexpf(mx, &e);  // e = 0 for a zero chunk
+      e = max(e, -100);
+      const float sc = ldexpf(1.0f, 15 - e);
+      if (live) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          f16x4 hi, lo;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float x = ot[j][4 * q + i] * sc;
+            hi[i] = static_cast<_Float16>(x);
+            lo[i] = static_cast<_Float16>(x - static_cast<float>(hi[i]));
+          }
+          *reinterpret_cast<f16x4*>(a.out_split.hi + row + 32 * j + 8 * q) = hi;
+          *reinterpret_cast<f16x4*>(a.out_split.lo + row + 32 * j + 8 * q) = lo;
+        }
+        if (half == 0)
+          a.out_split.inv[orow * (a.hq * D / kSplitChunkFine) + h * DT + j] = ldexpf(1.0f, e - 15);
+      }
+    }
+  }
 }
 
 // Block = 32 queries x kHeads query heads of one KV group; its 8 waves are 2
@@ -334,127 +433,354 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   }
   add_pv();
 
-  // Merge the key ranges pairwise: (m, l) per query, O^T as the lanes hold it.
-  float* mrg = reinterpret_cast<float*>(lds);
+  merge_and_write<D, HB>(a, ot, m_run, l_part, reinterpret_cast<float*>(lds), s, hb, lane, h, b, q0);
+}
+
+// The same over an fp32 cache, D = 64 or 96: block = 32 queries
+// x 4 query heads of one KV group, its 8 waves 4 heads x 2 key ranges.  K, V,
+// q and p all go to the matrix cores as hi + lo fp16 planes (22 bits; the lo x
+// lo products, 2^-22 of the others, are left out), with power-of-two scales
+// that keep every plane below 2^15: q per query, K and V per 8 keys, which are
+// the rows one wave stages and four of a lane's 16 scores, and p per 8 keys so
+// that O^T keeps one scale 2^(30 - E), E the largest V exponent so far.  K and
+// V pass through registers, where they are split, into the stage that the four
+// heads share.
+//
+// What bounds it: the matrix cores, 36 products of 32 cycles a tile and head
+// for d = 96 (1,152 cycles, where products of fp32 operands would take 6,144),
+// and the splits' and the softmax's vector instructions beside them.
+// prefill.hip's kernel / this one, 8 query heads on 2: d 96, 2,000 rows 118.9
+// / 88.5 us, 4,096 rows 398.5 / 171.1, 3,000 rows after 1,111 keys 349.9 /
+// 171.5; d 64 78.6 / 70.6, 249.6 / 136.9, 221.5 / 137.2.  Largest error
+// against 64 bits, of the largest value: d 96, 4,096 rows 3.5e-7 / 2.6e-7,
+// 3,000 rows after 3,000 keys 5.6e-7 / 3.4e-7 (a tile's values are summed
+// before they meet the long sums; added product by product it was 5.9e-7).
+constexpr int kHeads32 = 4;
+template <int D, bool kPool>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attention_f32_kernel(
+    PrefillAttnArgs a) {
+  constexpr int HB = kHeads32, S = kWaves / HB;
+  constexpr int kRow = D / 8;
+  constexpr int kPlaneBytes = kKeyTile * kRow * 16;
+  constexpr int kStageBytes = 4 * kPlaneBytes;  // K hi, K lo, V hi, V lo
+  constexpr int kMergeFloats = (D / 2 + 2) * kWave;
+  constexpr int kStages = 2 * S * kStageBytes;
+  constexpr int kLdsBytes = kStages > kMergeFloats * 4 * kWaves / 2 ? kStages : kMergeFloats * 4 * kWaves / 2;
+  constexpr int DJ = D / 16, DT = D / 32;
+  constexpr int kPer = D / 32;        // float4s of K (and of V) that a thread stages per tile
+  constexpr int kMinScoreExp = -40;  // smaller q or k count as 2^-40: their scores are 0 to fp32
+  __shared__ __align__(16) char lds[kLdsBytes];
+  __shared__ __align__(16) int k_exp[2][S][4], v_exp[2][S][4];
+
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int s = wave / HB, hb = wave % HB;
+  const int h = blockIdx.y * HB + hb;
+  const int g = h / (a.hq / a.hkv);
+  const int q0 = (gridDim.x - 1 - blockIdx.x) * kQueryTile;
+  const int qi = lane % 32, half = lane / 32;
+  const int qpos = a.start + q0 + qi;
+  const int b = blockIdx.z;
+  const int last_key = a.start + min(q0 + kQueryTile, a.tokens) - 1;
+  const int n_tiles = last_key / kKeyTile + 1;
+  const int n_iter = (n_tiles + S - 1) / S;
+
+  // This wave stages rows 8 hb .. + 7 of a tile: float4 lane + 64 i of them.
+  int srow[kPer], scol[kPer], spos[kPer];
 #pragma unroll
-  for (int step = S / 2; step >= 1; step /= 2) {
-    __syncthreads();  // the stages (or the previous round's values) have been read
-    if (s >= step && s < 2 * step) {
-      float* dst = mrg + ((s - step) * HB + hb) * kMergeFloats;
-#pragma unroll
-      for (int j = 0; j < DT; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<float4*>(dst + ((j * 4 + q) * kWave + lane) * 4) =
-              make_float4(ot[j][4 * q], ot[j][4 * q + 1], ot[j][4 * q + 2], ot[j][4 * q + 3]);
-      dst[D / 2 * kWave + lane] = m_run;
-      dst[D / 2 * kWave + kWave + lane] = l_part;
-    }
-    __syncthreads();
-    if (s < step) {
-      const float* src = mrg + (s * HB + hb) * kMergeFloats;
-      const float m_b = src[D / 2 * kWave + lane], l_b = src[D / 2 * kWave + kWave + lane];
-      const float m_new = fmaxf(m_run, m_b);
-      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-      const float ea = __builtin_amdgcn_exp2f(m_run - m_use), eb = __builtin_amdgcn_exp2f(m_b - m_use);
-      l_part = l_part * ea + l_b * eb;
-      m_run = m_new;
-#pragma unroll
-      for (int j = 0; j < DT; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4 v = *reinterpret_cast<const float4*>(src + ((j * 4 + q) * kWave + lane) * 4);
-          ot[j][4 * q] = fmaf(v.x, eb, ot[j][4 * q] * ea);
-          ot[j][4 * q + 1] = fmaf(v.y, eb, ot[j][4 * q + 1] * ea);
-          ot[j][4 * q + 2] = fmaf(v.z, eb, ot[j][4 * q + 2] * ea);
-          ot[j][4 * q + 3] = fmaf(v.w, eb, ot[j][4 * q + 3] * ea);
-        }
-    }
+  for (int i = 0; i < kPer; ++i) {
+    const int f = lane + i * kWave;
+    srow[i] = 8 * hb + f / (D / 4);
+    scol[i] = f % (D / 4) * 4;
+    spos[i] = tile_chunk<D>(srow[i], scol[i] / 8) * 16 + scol[i] % 8 * 2;
   }
-  if (s > 0) return;
-  const float inv = 1.0f / half_swap_sum(l_part);
-  const bool live = q0 + qi < a.tokens;
-  const int64_t orow = static_cast<int64_t>(b) * a.tokens + q0 + qi;
-  const int64_t row = orow * a.out_stride + h * D + 4 * half;
-#pragma unroll
-  for (int j = 0; j < DT; ++j) {
-    ot[j] *= inv;
-    if (a.out && live) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4*>(a.out + row + 32 * j + 8 * q) =
-            make_float4(ot[j][4 * q], ot[j][4 * q + 1], ot[j][4 * q + 2], ot[j][4 * q + 3]);
+  f32x4 kreg[kPer], vreg[kPer];
+  auto load = [&](f32x4 (&r)[kPer], void* const* seg_base, const void* pool, int i) {
+    const int t0 = min(s + i * S, n_tiles - 1) * kKeyTile;
+    const float* base;
+    if constexpr (kPool) {
+      base = static_cast<const float*>(pool) + kv_pool_offset(a.pool.interleave, b, t0, g, a.hkv, D);
+    } else {
+      const int seg = kv_segment(t0);
+      base = static_cast<const float*>(seg_base[2 * seg]) + kv_segment_offset(seg, t0, g, a.hkv, D);
     }
-    if (a.out_split.hi) {  // the 32 dims of slice j are one chunk: 16 here, 16 in the other half
-      float mx = 0.0f;
+    const int limit = last_key - t0;  // rows past the last key are masked, any key's row will do
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(ot[j][i]));
-      mx = half_swap_max(mx);
-      int e = 0;
-      frexpf(mx, &e);  // e = 0 for a zero chunk
-      e = max(e, -100);
-      const float sc = ldexpf(1.0f, 15 - e);
-      if (live) {
+    for (int u = 0; u < kPer; ++u) r[u] = *reinterpret_cast<const f32x4*>(base + min(srow[u], limit) * D + scol[u]);
+  };
+  static_assert(sizeof(KvSeg) == 2 * sizeof(void*), "segments are (k, v) pairs");
+  auto load_k = [&](int i) { load(kreg, &a.seg.s[0].k, a.pool.k, i); };
+  auto load_v = [&](int i) { load(vreg, &a.seg.s[0].v, a.pool.v, i); };
+  char* stage0 = lds + s * kStageBytes;
+  auto stage = [&](int parity) { return stage0 + parity * S * kStageBytes; };
+  // The wave's 8 rows to one exponent (at least `least`) and two planes.
+  auto store = [&](const f32x4 (&r)[kPer], char* hi_plane, int* exponent, int least) {
+    float mx = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          f16x4 hi, lo;
+    for (int u = 0; u < kPer; ++u)
+      mx = fmaxf(fmaxf(fmaxf(mx, fabsf(r[u][0])), fmaxf(fabsf(r[u][1]), fabsf(r[u][2]))), fabsf(r[u][3]));
+    mx = group_max<kWave>(mx);
+    const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx), least) : least;
+    const float sc = ldexpf(1.0f, 15 - e);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float x = ot[j][4 * q + i] * sc;
-            hi[i] = static_cast<_Float16>(x);
-            lo[i] = static_cast<_Float16>(x - static_cast<float>(hi[i]));
-          }
-          *reinterpret_cast<f16x4*>(a.out_split.hi + row + 32 * j + 8 * q) = hi;
-          *reinterpret_cast<f16x4*>(a.out_split.lo + row + 32 * j + 8 * q) = lo;
-        }
-        if (half == 0)
-          a.out_split.inv[orow * (a.hq * D / kSplitChunkFine) + h * DT + j] = ldexpf(1.0f, e - 15);
+    for (int u = 0; u < kPer; ++u) {
+      uint32_t hw[2], lw[2];
+#pragma unroll
+      for (int w = 0; w < 2; ++w) split2(r[u][2 * w] * sc, r[u][2 * w + 1] * sc, hw[w], lw[w]);
+      *reinterpret_cast<uint2*>(hi_plane + spos[u]) = make_uint2(hw[0], hw[1]);
+      *reinterpret_cast<uint2*>(hi_plane + kPlaneBytes + spos[u]) = make_uint2(lw[0], lw[1]);
+    }
+    if (lane == 0) exponent[hb] = e;
+  };
+  auto store_k = [&](int parity) { store(kreg, stage(parity), k_exp[parity][s], kMinScoreExp); };
+  auto store_v = [&](int parity) { store(vreg, stage(parity) + 2 * kPlaneBytes, v_exp[parity][s], -100); };
+  auto barrier = [&] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+  load_k(0);
+  load_v(0);
+
+  // Q^T: dims 16 j + 8 half + {0..7} of query qi times log2(e) / sqrt(d) and
+  // the query's scale 2^(15 - e_q), split hi + lo.
+  f16x8 qh[DJ], ql[DJ];
+  int e_q = kMinScoreExp;
+  {
+    const float qscale = 1.4426950408889634f / sqrtf(static_cast<float>(D));
+    const int64_t qrow = static_cast<int64_t>(b) * a.tokens + min(q0 + qi, a.tokens - 1);
+    const float* qsrc = a.query + qrow * a.query_stride + h * D + 8 * half;
+    float x[DJ][8];
+    float mx = 0.0f;
+#pragma unroll
+    for (int j = 0; j < DJ; ++j) {
+      const float4 x0 = *reinterpret_cast<const float4*>(qsrc + 16 * j);
+      const float4 x1 = *reinterpret_cast<const float4*>(qsrc + 16 * j + 4);
+      const float y[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[j][e] = y[e] * qscale;
+        mx = fmaxf(mx, fabsf(x[j][e]));
       }
     }
+    mx = half_swap_max(mx);
+    if (mx > 0.0f) e_q = max(__builtin_amdgcn_frexp_expf(mx), kMinScoreExp);
+    const float sc = ldexpf(1.0f, 15 - e_q);
+#pragma unroll
+    for (int j = 0; j < DJ; ++j) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[j][e] *= sc;
+      split8(x[j], qh[j], ql[j]);
+    }
   }
+
+  f32x16 ot[DT];  // O^T 2^(30 - e_run): [dim 32 jt + 8 (i / 4) + 4 half + i % 4][query qi]
+#pragma unroll
+  for (int j = 0; j < DT; ++j) ot[j] = f32x16{};
+  float m_run = -INFINITY, l_part = 0.0f, alpha = 1.0f;
+  int e_run = -100;
+  bool grew = false;  // wave-uniform
+
+  auto scores = [&](int parity) {
+    const char* kst = stage(parity);
+    f32x16 st{};
+#pragma unroll
+    for (int j = 0; j < DJ; ++j) {
+      const int pos = tile_chunk<D>(qi, 2 * j + half) * 16;
+      const f16x8 kh = *reinterpret_cast<const f16x8*>(kst + pos);
+      const f16x8 kl = *reinterpret_cast<const f16x8*>(kst + pos + kPlaneBytes);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[j], st, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[j], st, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[j], st, 0, 0, 0);
+    }
+    return st;
+  };
+  f16x8 ph[2], pl[2];
+  auto add_pv = [&](int parity) {
+    const char* vst = stage(parity) + 2 * kPlaneBytes + lane % 2 * 8;
+#pragma unroll
+    for (int jt = 0; jt < DT; ++jt) {
+      f32x16 sum{};  // the tile's, before O^T's: a sixth of the roundings at O^T's size
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int row = 16 * t + 4 * half + lane % 16 / 4;
+        const int chunk = 4 * jt + lane / 16 % 2 * 2 + lane % 4 / 2;
+        auto column = [&](int plane) {
+          const char* src = vst + plane * kPlaneBytes;
+          const i16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) i16x4*)(src + tile_chunk<D>(row, chunk) * 16));
+          const i16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) i16x4*)(src + tile_chunk<D>(row + 8, chunk) * 16));
+          return __builtin_bit_cast(f16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        const f16x8 vh = column(0), vl = column(1);
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph[t], sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[t], sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[t], sum, 0, 0, 0);
+      }
+      ot[jt] += sum;
+    }
+  };
+
+  // Steps as in the fp16 kernel: K is staged two tiles ahead and V with its
+  // tile, each from registers that were loaded a step earlier.
+  store_k(0);
+  load_k(1);
+  store_k(1);
+  load_k(2);
+  barrier();
+  f32x16 st = scores(0);
+  int4 kx = *reinterpret_cast<const int4*>(&k_exp[0][s][0]);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) ph[t] = pl[t] = f16x8{};
+
+  auto step = [&](int i, auto parity) {
+    constexpr int kParity = decltype(parity)::value;  // i % 2
+    barrier();
+    store_k(kParity);
+    store_v(kParity);
+    load_k(i + 3);
+    load_v(i + 1);
+    const int t0 = (s + i * S) * kKeyTile;
+    if (t0 + kKeyTile - 1 > a.start + q0) {  // wave-uniform: the tile reaches past the first query
+#pragma unroll
+      for (int e = 0; e < 16; ++e) st[e] = t0 + 8 * (e / 4) + 4 * half + e % 4 <= qpos ? st[e] : -INFINITY;
+    }
+    const float inv[4] = {ldexpf(1.0f, e_q + kx.x - 30), ldexpf(1.0f, e_q + kx.y - 30), ldexpf(1.0f, e_q + kx.z - 30),
+                          ldexpf(1.0f, e_q + kx.w - 30)};
+    float mx = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      mx = fmaxf(mx, fmaxf(fmaxf(st[4 * q], st[4 * q + 1]), fmaxf(st[4 * q + 2], st[4 * q + 3])) * inv[q]);
+    mx = half_swap_max(mx);
+    // Tile i - 1's rise of the maximum or of V's exponent reaches O^T before
+    // its values do.
+    if (grew) {
+#pragma unroll
+      for (int j = 0; j < DT; ++j) ot[j] *= alpha;
+    }
+    const float m_new = fmaxf(m_run, mx);
+    grew = __any(m_new > m_run);
+    // No key of this query yet: the exponents below are of -inf - 0.
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+    alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    m_run = m_new;
+    l_part *= alpha;
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
+    const f32x16 st_next = scores(kParity ^ 1);
+    kx = *reinterpret_cast<const int4*>(&k_exp[kParity ^ 1][s][0]);
+    if (i > 0) add_pv(kParity ^ 1);
+    const int4 vx = *reinterpret_cast<const int4*>(&v_exp[kParity][s][0]);
+    const int e_new = max(max(e_run, max(vx.x, vx.y)), max(vx.z, vx.w));
+    grew = grew || e_new != e_run;
+    alpha = ldexpf(alpha, e_run - e_new);
+    e_run = e_new;
+    const float cg[4] = {ldexpf(1.0f, 15 + vx.x - e_new), ldexpf(1.0f, 15 + vx.y - e_new),
+                         ldexpf(1.0f, 15 + vx.z - e_new), ldexpf(1.0f, 15 + vx.w - e_new)};
+    float p[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(st[e], inv[e / 4], -m_use));
+    l_part += sum16(p);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) p[e] *= cg[e / 4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) split8(p + 8 * t, ph[t], pl[t]);
+    st = st_next;
+    __builtin_amdgcn_s_setprio(0);
+  };
+  if (wave >= kWaves / 2) barrier();
+  for (int i = 0; i < n_iter; i += 2) {
+    step(i, std::integral_constant<int, 0>{});
+    if (i + 1 < n_iter) step(i + 1, std::integral_constant<int, 1>{});
+  }
+  if (wave < kWaves / 2) barrier();
+  if (grew) {
+#pragma unroll
+    for (int j = 0; j < DT; ++j) ot[j] *= alpha;
+  }
+  add_pv((n_iter - 1) & 1);
+  const float unit = ldexpf(1.0f, e_run - 30);
+#pragma unroll
+  for (int j = 0; j < DT; ++j) ot[j] *= unit;
+  merge_and_write<D, HB>(a, ot, m_run, l_part, reinterpret_cast<float*>(lds), s, hb, lane, h, b, q0);
 }
 
 }  // namespace
 
-// Enough rows for this kernel, against prefill.hip's, whose blocks are 16
-// queries x 1 head, one per CU.  That one's time steps up when its blocks
-// pass 256, the CUs (512 rows for 8 heads); this one has a quarter as many
-// blocks, with a longer start and end, and wins once they fill about half the
-// CUs, or sooner after a long cached context, where the key loop is most of
-// the time.  d 96 (16-query kernel / this one): 512 rows 8.9 / 13.3 us, 700
-// rows 15.2 / 15.7, 1,000 rows 22.2 / 18.0; after 2,000 cached keys 300 rows
-// 21.9 / 28.3, 700 rows 43.7 / 32.5.  d 64: 700 rows 11.4 / 12.5, 1,000 rows
-// 15.1 / 14.6; after 2,000 keys 700 rows 30.2 / 26.3.  (d 128 does not fit
-// the registers of two waves per SIMD.)
-bool prefill_attention_many_rows(const PrefillAttnArgs& a) {
-  if (a.d != 32 && a.d != 64 && a.d != 96) return false;
+// What both kernels need: rows are read and written 16 bytes at a time, and a
+// block's heads are of one KV group.
+static bool many_rows_shape(const PrefillAttnArgs& a, int heads) {
   if ((reinterpret_cast<uintptr_t>(a.query) | reinterpret_cast<uintptr_t>(a.out)) % 16 != 0 ||
       (a.query_stride | a.out_stride) % 4 != 0)
-    return false;  // rows are read and written 16 bytes at a time
-  if (a.hkv <= 0 || a.hq % a.hkv != 0 || a.hq / a.hkv % kHeads != 0) return false;
-  const int64_t blocks = int64_t{(a.tokens + kQueryTile - 1) / kQueryTile} * (a.hq / kHeads) * a.seqs;
-  return blocks >= 112 || (blocks >= 80 && a.start >= a.tokens);
+    return false;
+  return a.hkv > 0 && a.hq % a.hkv == 0 && a.hq / a.hkv % heads == 0;
+}
+static int64_t many_rows_blocks(const PrefillAttnArgs& a, int heads) {
+  return int64_t{(a.tokens + kQueryTile - 1) / kQueryTile} * (a.hq / heads) * a.seqs;
+}
+
+// Enough rows for these kernels, against prefill.hip's, whose blocks are 16
+// queries x 1 head, one per CU.
+//
+// fp16 cache: that one's time steps up when its blocks pass 256, the CUs (512
+// rows for 8 heads); this one has a quarter as many blocks, with a longer start
+// and end, and wins once they fill about half the CUs, or sooner after a long
+// cached context, where the key loop is most of the time.  d 96 (16-query
+// kernel / this one): 512 rows 8.9 / 13.3 us, 700 rows 15.2 / 15.7, 1,000 rows
+// 22.2 / 18.0; after 2,000 cached keys 300 rows 21.9 / 28.3, 700 rows 43.7 /
+// 32.5.  d 64: 700 rows 11.4 / 12.5, 1,000 rows 15.1 / 14.6; after 2,000 keys
+// 700 rows 30.2 / 26.3.  (d 128 does not fit the registers of two waves per
+// SIMD.)
+//
+// fp32 cache: an eighth as many blocks.  8 heads, d 96: 1,000 rows (64 blocks)
+// 43.8 / 49.8, 2,000 rows (126) 118.9 / 88.5; after 2,000 keys 1,000 rows 114.2
+// / 126.3.  d 64: 1,000 rows 29.3 / 40.3, 2,000 rows 78.6 / 70.6; after 2,000
+// keys 1,000 rows 74.6 / 100.9.  (d 32, with a third of d 96's products to the
+// same softmax and splits, measured slower at all but 4,096 rows.)
+bool prefill_attention_many_rows(const PrefillAttnArgs& a, KvDtype kv) {
+  if (kv == kKvF16) {
+    if ((a.d != 32 && a.d != 64 && a.d != 96) || !many_rows_shape(a, kHeads)) return false;
+    const int64_t blocks = many_rows_blocks(a, kHeads);
+    return blocks >= 112 || (blocks >= 80 && a.start >= a.tokens);
+  }
+  return kv == kKvF32 && (a.d == 64 || a.d == 96) && many_rows_shape(a, kHeads32) &&
+         many_rows_blocks(a, kHeads32) >= 120;
 }
 
 namespace {
+// The page lookup is a compile-time choice: a branch there would cut the
+// step's matrix products into two blocks (82 -> 93 us a pass, fp16, 3,000 rows).
 template <int D>
-void launch_many_rows(const PrefillAttnArgs& a, hipStream_t stream) {
+void launch_f16(const PrefillAttnArgs& a, hipStream_t stream) {
   const dim3 grid((a.tokens + kQueryTile - 1) / kQueryTile, a.hq / kHeads, a.seqs);
-  // The page lookup is a compile-time choice: a branch there would cut the
-  // step's matrix products into two blocks (82 -> 93 us a pass, 3,000 rows).
   if (a.pool.k) {
     prefill_attention_f16_kernel<D, true><<<grid, kThreads, 0, stream>>>(a);
   } else {
     prefill_attention_f16_kernel<D, false><<<grid, kThreads, 0, stream>>>(a);
   }
 }
+template <int D>
+void launch_f32(const PrefillAttnArgs& a, hipStream_t stream) {
+  const dim3 grid((a.tokens + kQueryTile - 1) / kQueryTile, a.hq / kHeads32, a.seqs);
+  if (a.pool.k) {
+    prefill_attention_f32_kernel<D, true><<<grid, kThreads, 0, stream>>>(a);
+  } else {
+    prefill_attention_f32_kernel<D, false><<<grid, kThreads, 0, stream>>>(a);
+  }
+}
 }  // namespace
 
-hipError_t launch_prefill_attention_many_rows(const PrefillAttnArgs& a, hipStream_t stream) {
+hipError_t launch_prefill_attention_many_rows(const PrefillAttnArgs& a, KvDtype kv, hipStream_t stream) {
+  if (kv == kKvF32) {
+    switch (a.d) {
+      case 64: launch_f32<64>(a, stream); break;
+      case 96: launch_f32<96>(a, stream); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   switch (a.d) {
-    case 32: launch_many_rows<32>(a, stream); break;
-    case 64: launch_many_rows<64>(a, stream); break;
-    case 96: launch_many_rows<96>(a, stream); break;
+    case 32: launch_f16<32>(a, stream); break;
+    case 64: launch_f16<64>(a, stream); break;
+    case 96: launch_f16<96>(a, stream); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

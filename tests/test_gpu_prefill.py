@@ -203,6 +203,47 @@ def test_prefill_attention_many_rows(gpu, d, hq, hkv, start, T):
         assert rel_err(got[:, h], ref) < 1e-5, h
 
 
+@pytest.mark.parametrize("d", [64, 96])
+@pytest.mark.parametrize("hq,hkv,start,T,spread", [(32, 8, 0, 449, 0), (32, 4, 37, 480, 0), (16, 2, 1000, 993, 8),
+                                                   (16, 4, 511, 961, 14)])
+def test_prefill_attention_many_rows_f32(gpu, d, hq, hkv, start, T, spread):
+    # the 32-query kernel over an fp32 cache: a last query tile of 1, 32, 1 and
+    # 1 rows, groups of 4, 8, 8 and 4 heads, a context that crosses segments.
+    # With a spread, V grows with the position by 2^spread and falls again, so
+    # that the values' running scale moves, and K's rows (and, inversely, the
+    # queries) differ in size.  Against 64 bits: K, V, q and p carry 22 bits
+    # (2.4e-7 each; a score of size 10 turns two of these into 3.4e-6 of p at
+    # most, averaged over the keys) and sums are fp32 over tiles of 32 keys:
+    # 2e-6 of the largest value of the row, where one wrong key among 1,993 is
+    # about 1e-2.
+    mmr = gpu
+    print(f"[case] prefill attention many rows f32 d={d} hq={hq} hkv={hkv} start={start} T={T}", flush=True)
+    rng = np.random.default_rng(d + hq + start + T)
+    n = start + T
+    k = rng.standard_normal((hkv, n, d)).astype(np.float32)
+    v = rng.standard_normal((hkv, n, d)).astype(np.float32)
+    q = rng.standard_normal((T, hq, d)).astype(np.float32)
+    size = 2.0 ** (spread * (1 - np.abs(np.linspace(-1, 1, n))))
+    v *= size[None, :, None].astype(np.float32)
+    k *= np.float32(2.0**-spread)
+    k[:, ::3] *= np.float32(0.25)
+    q *= np.float32(2.0**spread)
+    cache = mmr.KvCache(hkv, d, n, mmr.KV_F32)
+    cache.upload(k, v)
+    dq, out = mmr.DeviceArray.from_numpy(q.reshape(T, hq * d)), mmr.DeviceArray((T, hq * d), np.float32)
+    mmr.prefill_attention(dq, cache, start, T, hq, hkv, d, out)
+    got = out.numpy().reshape(T, hq, d)
+    hidden = np.arange(n)[None, :] > start + np.arange(T)[:, None]
+    for h in range(hq):
+        g = h // (hq // hkv)
+        s = q[:, h].astype(np.float64) @ k[g].astype(np.float64).T / np.sqrt(d)
+        s[hidden] = -np.inf
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        ref = p @ v[g].astype(np.float64) / p.sum(axis=1, keepdims=True)
+        err = np.abs(got[:, h] - ref).max(axis=1) / np.abs(ref).max(axis=1)
+        assert err.max() < 2e-6, (h, int(err.argmax()), float(err.max()))
+
+
 def synth_model(mmr, g):
     return mmr.Model.synthetic(mmr.make_config(**g["config"]), g["seed"], g["std"], g["round_fp16"])
 
