@@ -6,6 +6,7 @@
 #include "device_common.h"
 #include "kernels.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace mmr {
@@ -25,7 +26,7 @@ constexpr int kActLd = kBN / 2 + 4;                            // floats per row
 static_assert(kBM * kActLd * 4 <= kStages * kStageBytes, "act tile exceeds the stages");
 
 enum : int { kA32, kAPlanes };  // fp32 rows; fp16 planes with one scale per row
-enum : int { kStore, kResidual, kSwiGlu };
+enum : int { kStore, kStoreSplit, kResidual, kSwiGlu };  // kStoreSplit: K split over gridDim.z
 
 // 16-byte chunk position of (row, chunk) in a stage [rows][8 chunks]: the 16
 // rows that a fragment read takes at one chunk lie in 16 distinct 16-byte
@@ -45,7 +46,8 @@ __device__ __forceinline__ int chunk_pos(int row, int chunk) { return row * kRow
 // 36.2 us (447 -> 712 TFLOP/s of products); 4,096 rows 106 -> 67 us; pre-split
 // A, 6,000 rows: gate_up + SwiGLU 109 -> 85 us, QKV 39 -> 29 us.  (128 x 128
 // tiles of 4 waves, two blocks per CU: 101 and 36 us; 64 x 128 per wave with
-// one level of sums: 96 us and twice the error.)
+// one level of sums: 96 us and twice the error.)  K may be split over
+// gridDim.z (gemm_rows_splits).
 template <int kA, int kEpi>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_kernel(GemmArgs g) {
   __shared__ __align__(16) char lds[kStages * kStageBytes];
@@ -66,7 +68,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int band = tile / (8 * nt), in_band = tile % (8 * nt);
   const int band_rows = min(8, mt - band * 8);
   const int m0 = (band * 8 + in_band % band_rows) * kBM, n0 = in_band / band_rows * kBN;
-  const int nk = g.k / kBK;  // even
+  int nk = g.k / kBK;  // even
+  if constexpr (kEpi == kStoreSplit) {
+    // Split z of S takes pairs of stages z P / S .. (z + 1) P / S of the P =
+    // K / 128, at least one; the operands and the output start there.
+    const int pairs = nk / 2, split = static_cast<int>(blockIdx.z), splits = static_cast<int>(gridDim.z);
+    const int first = pairs * split / splits;
+    nk = 2 * (pairs * (split + 1) / splits - first);
+    g.w += first * 2 * kBK;
+    if constexpr (kA == kA32) {
+      g.a += first * 2 * kBK;
+    } else {
+      g.a_hi += first * 2 * kBK;
+      g.a_lo += first * 2 * kBK;
+    }
+    g.c += split * g.split_stride;
+  }
 
   // Direct loads: wave-wide load i fills rows 8 i .. + 7 of a plane (128 bytes
   // each: whole cache lines); this wave takes loads wave, wave + 8, ...
@@ -345,8 +362,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 template <int kA>
 void launch(const GemmArgs& g, hipStream_t s) {
   const int tiles = ((g.m + kBM - 1) / kBM) * ((g.n + kBN - 1) / kBN);
-  const int grid = (tiles + kXcds - 1) / kXcds * kXcds;
-  if (g.swiglu) {
+  const dim3 grid((tiles + kXcds - 1) / kXcds * kXcds, 1, g.k_splits);  // x % 8 == 0: a tile's splits share an XCD
+  if (g.k_splits > 1) {
+    gemm_rows_kernel<kA, kStoreSplit><<<grid, kThreads, 0, s>>>(g);
+  } else if (g.swiglu) {
     gemm_rows_kernel<kA, kSwiGlu><<<grid, kThreads, 0, s>>>(g);
   } else if (g.residual) {
     gemm_rows_kernel<kA, kResidual><<<grid, kThreads, 0, s>>>(g);
@@ -357,7 +376,28 @@ void launch(const GemmArgs& g, hipStream_t s) {
 
 }  // namespace
 
-// Tiles of this kernel enough for it, against prefill.hip's smaller ones: a
+// K splits for a launch of too few tiles for the chip (the plain products of
+// the prefill layers, whose consumers add the partials): up to 3, as many as
+// keep the blocks to one round, each XCD's 32 CUs taking its share of the tiles
+// times the splits.  Whole prompts (fp16 cache, MiniMind2, tiles of O and down
+// / of QKV; before: 64 x 64 tiles for O and down, QKV unsplit): 2,500 tokens,
+// 60 / 100 tiles, 3 and 2 splits, 3.79 -> 3.57 ms (QKV unsplit 3.64); 3,000
+// tokens, 72 / 120, 4.33 -> 3.93 (2 and 2 splits: 4.12); 3,500 tokens, 84, 2
+// splits, 4.62 -> 4.51 (3, whose 33 blocks an XCD are two rounds: 4.77); 4,096
+// tokens, 96, 2 splits, 5.20 -> 5.01; 2,300 tokens, 54, 3.47 -> 3.34; but 2,048
+// tokens, 48 tiles, 2.88 -> 2.94.  4 splits (60 tiles) equal 3; fewer rows are
+// not worth it (900 rows, 24 tiles, 8 splits: 1.90 -> 2.01 ms), nor is a short
+// K (QKV of 2,500 x 768 x 512 in 3 splits: small model 1.25 -> 1.28 ms).
+int gemm_rows_splits(int m, int n, int k) {
+  constexpr int kMinRows = 1024, kMinTiles = 54, kMinK = 768, kMaxSplits = 3, kXcdCus = 32;
+  if (m < kMinRows || k < kMinK || k % (2 * kBK) != 0) return 0;
+  const int64_t tiles = static_cast<int64_t>((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
+  const int64_t per_xcd = (tiles + kXcds - 1) / kXcds;
+  const int64_t splits = std::min<int64_t>(kMaxSplits, kXcdCus / per_xcd);
+  return tiles >= kMinTiles && splits > 1 ? static_cast<int>(splits) : 0;
+}
+
+// Tiles of this kernel enough for it unsplit, against prefill.hip's smaller ones: a
 // block takes a CU to itself, so a launch takes as long as one block per
 // round of 256, and from 96 tiles on that is the shorter (fp32 A, prefill.hip
 // / this one: 88 tiles, 1,000 rows of 2816 x 512, 24.4 / 22.3 us; 96 tiles,
@@ -366,9 +406,11 @@ void launch(const GemmArgs& g, hipStream_t s) {
 // 1,000 rows of 4096 x 768, 33.3 / 33.3; 352 tiles, 4,096 rows of 2816 x 512,
 // 59.9 / 44.8).
 bool gemm_many_rows(const GemmArgs& g) {
+  constexpr int kMinTiles = 96;
   const int64_t a_bytes = static_cast<int64_t>(g.m) * g.lda * 2, w_bytes = static_cast<int64_t>(g.n) * g.k * 2;
   const int64_t tiles = static_cast<int64_t>((g.m + kBM - 1) / kBM) * ((g.n + kBN - 1) / kBN);
-  return tiles >= 96 && tiles < (1 << 30) && g.k_splits == 1 && !g.register_staged && g.k % (2 * kBK) == 0 &&
+  const bool enough = g.k_splits == 1 ? tiles >= kMinTiles : g.k_splits == gemm_rows_splits(g.m, g.n, g.k);
+  return enough && tiles < (1 << 30) && !g.register_staged && g.k % (2 * kBK) == 0 &&
          (!g.a_hi || g.a_chunk == kSplitChunk) && (!g.swiglu || (g.n % 8 == 0 && g.ldc % 4 == 0)) &&
          (reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.a_hi) | reinterpret_cast<uintptr_t>(g.a_lo) |
           reinterpret_cast<uintptr_t>(g.w)) % 16 == 0 &&

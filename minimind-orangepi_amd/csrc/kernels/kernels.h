@@ -328,7 +328,8 @@ struct GemmArgs {
 };
 bool gemm_supported(int m, int n, int k);
 // Split count launch_gemm accepts and uses well for this shape: about four
-// 128-wide K tiles per split; 1 where the few-rows path applies.
+// 128-wide K tiles per split, for many rows gemm_rows_splits; 1 where the
+// few-rows path applies.
 int gemm_k_splits(int m, int n, int k);
 // Whether launch_gemm takes the SwiGLU epilogue for this shape (unsplit tiles).
 bool gemm_swiglu_supported(int m, int n, int k);
@@ -344,6 +345,9 @@ hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
 // The kernel for many rows (gemm_rows.hip), which launch_gemm takes where it
 // is the faster one.
 bool gemm_many_rows(const GemmArgs& g);
+// K splits with which that kernel serves a plain product of fp32 rows or of
+// planes per 128 columns; 0: its unsplit launch or the other kernels.
+int gemm_rows_splits(int m, int n, int k);
 hipError_t launch_gemm_many_rows(const GemmArgs& g, hipStream_t stream);
 
 // A batch's KV page pools ([page][Hkv][kKvPage][D], see AttnArgs): page p of

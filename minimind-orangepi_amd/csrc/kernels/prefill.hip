@@ -1238,6 +1238,7 @@ GemmTiling choose_gemm_tiling(int m, int n, int k) {
 
 int gemm_k_splits(int m, int n, int k) {
   if (!gemm_supported(m, n, k) || use_skinny(m, k)) return 1;
+  if (const int rows_splits = gemm_rows_splits(m, n, k)) return rows_splits;
   return choose_gemm_tiling(m, n, k).splits;
 }
 

@@ -62,9 +62,12 @@ SplitChoice split_choice(const MiniMindConfig& c, int rows) {
   sc.x = mmr::gemm_presplit_supported(rows, qkv_w, H) && mmr::gemm_presplit_supported(rows, 2 * F, H);
   // Likewise the attention output (written split by the attention kernel)
   // for the O GEMM, and act (written split by the gate_up SwiGLU epilogue)
-  // for the down GEMM.
-  sc.attn = D % mmr::kSplitChunkFine == 0 && mmr::gemm_presplit_supported(rows, H, Hq * D);
-  sc.act = mmr::gemm_swiglu_split_supported(rows, 2 * F, H) && mmr::gemm_presplit_supported(rows, H, F);
+  // for the down GEMM; where the many-rows kernel takes those, it splits their
+  // fp32 rows itself.
+  sc.attn = D % mmr::kSplitChunkFine == 0 && mmr::gemm_presplit_supported(rows, H, Hq * D) &&
+            mmr::gemm_rows_splits(rows, H, Hq * D) == 0;
+  sc.act = mmr::gemm_swiglu_split_supported(rows, 2 * F, H) && mmr::gemm_presplit_supported(rows, H, F) &&
+           mmr::gemm_rows_splits(rows, H, F) == 0;
   return sc;
 }
 

@@ -6,7 +6,8 @@
 // attention -> O GEMM + residual -> RMSNorm rows -> gate_up GEMM + SwiGLU ->
 // down GEMM + residual, on the fp16 matrix cores (kernels/prefill.hip), over a
 // residual stream updated in place.  The whole-model prefill runs it layer
-// after layer on 512-row chunks; the C ABI runs one layer on a caller's rows.
+// after layer on passes of up to 4,096 rows; the C ABI runs one layer on a
+// caller's rows.
 // Nothing here allocates or synchronises: every buffer comes from a
 // PrefillScratch carved out of memory the caller owns.
 #pragma once

@@ -352,10 +352,12 @@ def test_minimind2_ragged_chunks_match_tokenwise(gpu, monkeypatch, prompt_len):
     assert gem.read_sequence(prompt_len, 1).tolist() == tok.read_sequence(prompt_len, 1).tolist()
 
 
-@pytest.mark.parametrize("prompt_len", [2500, 5000])
+@pytest.mark.parametrize("prompt_len", [2305, 2500, 3500, 5000])
 def test_minimind2_long_passes_match_chunks(gpu, monkeypatch, prompt_len):
-    # one pass of 2,500 rows and two of them (the many-rows GEMM for QKV and
-    # gate_up, the many-rows attention after 2,500 cached rows) against the
+    # one pass of 2,500 rows and two of them (the many-rows GEMM for every
+    # projection, O and down in 3 K splits, QKV in 2; the many-rows attention
+    # after 2,500 cached rows), 2,305 (a last row tile of 1 row, K in uneven
+    # splits of 5, 5 and 6 chunks) and 3,500 (2 splits, QKV 1) against the
     # same prompt in 512-row chunks: same next token, logits within 1e-4 (fp16
     # K/V roundings of differently grouped fp32 sums, as in the tests below)
     mmr = gpu

@@ -192,6 +192,21 @@ def test_prefill_partial_buffer_covers_every_chunk_row_count(mmr, case):
     assert mmr.prefill_partial_floats(cfg, 0) == 0
 
 
+def test_many_rows_splits_fill_one_round_and_leave_no_split_empty(mmr):
+    # From 54 tiles of 128 x 256 on, a product of at least 1,024 rows and 768 columns is split
+    # along K: every split has a 128-column chunk, and an XCD's share of the
+    # tiles times the splits stays within its 32 CUs.
+    for n, k in [(768, 2048), (768, 768), (1152, 768), (512, 1408), (1536, 896), (300, 1024), (768, 832)]:
+        for m in (1023, 1024, 2303, 2304, 2305, 2500, 3328, 3329, 3500, 4096, 20000):
+            tiles = -(-m // 128) * -(-n // 256)
+            splits = mmr.gemm_k_splits(m, n, k)
+            if m < 1024 or k % 128 or k < 768 or tiles < 54:
+                continue
+            assert 1 <= splits <= 3 and splits <= k // 128
+            assert splits == 1 or -(-tiles // 8) * splits <= 32, (m, n, k, splits)
+    assert [mmr.gemm_k_splits(m, 768, 2048) for m in (2500, 3000, 3500, 4096)] == [3, 3, 2, 2]
+
+
 @pytest.mark.parametrize("head_dim,tile", [(96, 64), (64, 64), (128, 32)])
 def test_decode_split_buckets(mmr, head_dim, tile):
     # The decode step replays one graph per attention split count, and the KV
