@@ -99,6 +99,9 @@ int mmr_launch_floor_us(int kernels, int blocks, int load_store, int reps, float
  * 1..chunk_rows). */
 int mmr_gemm_k_splits(int64_t m, int64_t n, int64_t k, int* splits);
 int mmr_prefill_partial_floats(const mmr_config* config, int64_t chunk_rows, int64_t* floats);
+/* Test aid, no reference counterpart (host arithmetic, no device needed):
+ * whether an unsplit m x n x k product takes the 128 x 256 tiles for many rows. */
+int mmr_gemm_many_rows(int64_t m, int64_t n, int64_t k, int* many_rows);
 /* Test aid, no reference counterpart: the (W row block, K chunk) that block
  * `block` of a batched split-K GEMM launch with grid (row_blocks, chunks)
  * computes (the blocks of one K chunk are placed on one XCD where chunks is a

@@ -285,6 +285,13 @@ int mmr_gemm_k_splits(int64_t m, int64_t n, int64_t k, int* splits) {
     *splits = mmr::gemm_k_splits(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
   });
 }
+int mmr_gemm_many_rows(int64_t m, int64_t n, int64_t k, int* many_rows) {
+  return guarded([&] {
+    require(many_rows, "null result");
+    require(m > 0 && n > 0 && k > 0 && m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX, "shape out of range");
+    *many_rows = mmr::gemm_rows_unsplit(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
+  });
+}
 int mmr_splitk_block_tile(int block, int row_blocks, int chunks, int* row_block, int* chunk) {
   return guarded([&] {
     require(row_block && chunk, "null argument");

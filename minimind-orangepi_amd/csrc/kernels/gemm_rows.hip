@@ -397,19 +397,34 @@ int gemm_rows_splits(int m, int n, int k) {
   return tiles >= kMinTiles && splits > 1 ? static_cast<int>(splits) : 0;
 }
 
-// Tiles of this kernel enough for it unsplit, against prefill.hip's smaller ones: a
-// block takes a CU to itself, so a launch takes as long as one block per
-// round of 256, and from 96 tiles on that is the shorter (fp32 A, prefill.hip
-// / this one: 88 tiles, 1,000 rows of 2816 x 512, 24.4 / 22.3 us; 96 tiles,
-// 4,096 rows of 768 x 2048, 77.0 / 72.2; 80 tiles, 2,048 rows of 1152 x 768,
-// 32.1 / 30.3; 64 tiles, 4,096 rows of 512 x 1408, 46.2 / 51.9; 128 tiles,
-// 1,000 rows of 4096 x 768, 33.3 / 33.3; 352 tiles, 4,096 rows of 2816 x 512,
-// 59.9 / 44.8).
+// The unsplit launch against prefill.hip's kernels: a block takes a CU to
+// itself, so a launch takes as long as one block per round of 256, and from 96
+// tiles on that is the shorter (fp32 A, prefill.hip / this one: 88 tiles, 1,000
+// rows of 2816 x 512, 24.4 / 22.3 us; 96 tiles, 4,096 rows of 768 x 2048, 77.0 /
+// 72.2; 80 tiles, 2,048 rows of 1152 x 768, 32.1 / 30.3; 64 tiles, 4,096 rows of
+// 512 x 1408, 46.2 / 51.9; 128 tiles, 1,000 rows of 4096 x 768, 33.3 / 33.3; 352
+// tiles, 4,096 rows of 2816 x 512, 59.9 / 44.8).  A tile's rows must be there:
+// up to 64, one row of 64-row tiles does the same product on finer blocks (64
+// rows of 24576 x 768 20.3 / 27.5 us, of 24576 x 2048 42.4 / 64.1, of 32768 x
+// 768 25.4 / 28.4; 65 rows of 24576 x 256, 768, 2048 and 4096 15.6 / 12.8, 30.9 /
+// 27.7, 68.8 / 64.0 and 128.4 / 122.8).  Of the few-rows kernel's range (up to
+// 32 rows, K >= 256) that one keeps up to 16 rows (8 rows of 32768 x 768 18.7 /
+// 27.0) and, for 17-32, launches below 160 tiles (17 rows of 24576 x 768 21.9 /
+// 26.3, of 24576 x 4096 79.8 / 121.6; but of 49152 x 512, 192 tiles, 39.4 /
+// 21.9, of 65536 x 768, 256 tiles, 52.5 / 32.4 and of 151936 x 1024, 594 tiles,
+// 128.3 / 115.4).
+bool gemm_rows_unsplit(int m, int n, int k) {
+  constexpr int kMinTiles = 96, kMinRows = 65, kFewRows = 17, kFewRowsEnd = 32, kFewRowsTiles = 160, kFewRowsK = 256;
+  const int64_t tiles = static_cast<int64_t>((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
+  if (k % (2 * kBK) != 0) return false;
+  if (m >= kFewRows && m <= kFewRowsEnd) return k >= kFewRowsK && tiles >= kFewRowsTiles;
+  return m >= kMinRows && tiles >= kMinTiles;
+}
+
 bool gemm_many_rows(const GemmArgs& g) {
-  constexpr int kMinTiles = 96;
   const int64_t a_bytes = static_cast<int64_t>(g.m) * g.lda * 2, w_bytes = static_cast<int64_t>(g.n) * g.k * 2;
   const int64_t tiles = static_cast<int64_t>((g.m + kBM - 1) / kBM) * ((g.n + kBN - 1) / kBN);
-  const bool enough = g.k_splits == 1 ? tiles >= kMinTiles : g.k_splits == gemm_rows_splits(g.m, g.n, g.k);
+  const bool enough = g.k_splits == 1 ? gemm_rows_unsplit(g.m, g.n, g.k) : g.k_splits == gemm_rows_splits(g.m, g.n, g.k);
   return enough && tiles < (1 << 30) && !g.register_staged && g.k % (2 * kBK) == 0 &&
          (!g.a_hi || g.a_chunk == kSplitChunk) && (!g.swiglu || (g.n % 8 == 0 && g.ldc % 4 == 0)) &&
          (reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.a_hi) | reinterpret_cast<uintptr_t>(g.a_lo) |

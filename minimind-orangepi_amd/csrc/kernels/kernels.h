@@ -345,6 +345,8 @@ hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
 // The kernel for many rows (gemm_rows.hip), which launch_gemm takes where it
 // is the faster one.
 bool gemm_many_rows(const GemmArgs& g);
+// Whether that kernel is the faster one for an unsplit product.
+bool gemm_rows_unsplit(int m, int n, int k);
 // K splits with which that kernel serves a plain product of fp32 rows or of
 // planes per 128 columns; 0: its unsplit launch or the other kernels.
 int gemm_rows_splits(int m, int n, int k);

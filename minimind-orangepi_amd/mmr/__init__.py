@@ -102,6 +102,7 @@ _SIGS = {
     "mmr_event_record": ([VP, VP], C.c_int),
     "mmr_event_elapsed_ms": ([VP, VP, P_F32], C.c_int),
     "mmr_gemm_k_splits": ([I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
+    "mmr_gemm_many_rows": ([I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
     "mmr_prefill_partial_floats": ([C.POINTER(Config), I64, C.POINTER(I64)], C.c_int),
     "mmr_splitk_block_tile": ([C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)], C.c_int),
     "mmr_decode_attention_splits": ([I64, I64, C.POINTER(C.c_int)], C.c_int),
@@ -373,6 +374,13 @@ def gemm_k_splits(m: int, n: int, k: int) -> int:
     out = C.c_int()
     check(_lib.mmr_gemm_k_splits(m, n, k, C.byref(out)))
     return out.value
+
+
+def gemm_many_rows(m: int, n: int, k: int) -> bool:
+    """Whether an unsplit m x n x k product takes the 128 x 256 tiles for many rows (host arithmetic)."""
+    out = C.c_int()
+    check(_lib.mmr_gemm_many_rows(m, n, k, C.byref(out)))
+    return bool(out.value)
 
 
 def splitk_block_tile(block: int, row_blocks: int, chunks: int) -> tuple[int, int]:

@@ -83,6 +83,22 @@ def test_matmul_many_rows_matches_fp64(gpu, batch, rows, cols, grow):
         assert rel_err(dr.numpy(), res + exact) < 1e-5
 
 
+@pytest.mark.parametrize("batch", [16, 17, 32, 33, 64, 65])
+def test_matmul_few_rows_wide_output_matches_fp64(gpu, batch):
+    # 160 tiles of 128 x 256 with few of their rows: the edges between the
+    # few-rows kernel, the 64-row tiles and the many-rows ones
+    mmr = gpu
+    rows, cols = 40960, 256
+    print(f"[case] matmul wide {batch}x{rows}x{cols}", flush=True)
+    rng = np.random.default_rng(batch)
+    w16, w32 = f16_weights(rng, rows, cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    dw, dx = mmr.DeviceArray.from_numpy(w16.view(np.uint16)), mmr.DeviceArray.from_numpy(x)
+    dy = mmr.DeviceArray((batch, rows), np.float32)
+    mmr.matmul_f16(dw, rows, cols, dx, batch, dy)
+    assert rel_err(dy.numpy(), x.astype(np.float64) @ w32.astype(np.float64).T) < 1e-5
+
+
 def test_matmul_rejects_bad_shapes(gpu):
     mmr = gpu
     d = mmr.DeviceArray(64, np.float32)

@@ -207,6 +207,20 @@ def test_many_rows_splits_fill_one_round_and_leave_no_split_empty(mmr):
     assert [mmr.gemm_k_splits(m, 768, 2048) for m in (2500, 3000, 3500, 4096)] == [3, 3, 2, 2]
 
 
+@pytest.mark.parametrize("m,n,k,chosen", [
+    (1, 65536, 768, False), (8, 32768, 768, False), (16, 65536, 768, False),  # the few-rows kernel
+    (17, 24576, 768, False), (32, 32768, 2048, False), (17, 40960, 768, True), (32, 65536, 768, True),
+    (32, 65536, 128, False),  # K below the few-rows kernel's: 32 x 64 tiles
+    (33, 24576, 768, False), (64, 65536, 768, False), (64, 151936, 1024, False),  # one row of 64-row tiles
+    (65, 24576, 768, True), (65, 24320, 768, False), (512, 6400, 768, True), (1000, 2816, 512, False),
+    (2048, 4096, 768, True), (2048, 4096, 832, False)])
+def test_many_rows_tiles_need_rows_as_well_as_tiles(mmr, m, n, k, chosen):
+    # 128 x 256 tiles from 96 of them on, but not where most of a tile's 128
+    # rows would be padding: few rows on a wide output (a batch's vocabulary
+    # projection) stay with the kernels written for them.
+    assert mmr.gemm_many_rows(m, n, k) is chosen
+
+
 @pytest.mark.parametrize("head_dim,tile", [(96, 64), (64, 64), (128, 32)])
 def test_decode_split_buckets(mmr, head_dim, tile):
     # The decode step replays one graph per attention split count, and the KV
