@@ -424,34 +424,30 @@ __device__ inline T sum_parts4(const T* part4, int64_t sstride, int s0, int step
 constexpr int kResChunkQuads = 256;
 constexpr int kResManyRows = 64;
 
-// The exponent e of a row's largest |value| = f 2^e, f in [1/2, 1): its planes'
-// scale is s = 2^(15 - e).  One scale serves the whole row (every chunk's inv
-// holds the same 1 / s): fp16 keeps 11 bits of each plane at any magnitude, so
-// hi + lo has its 22 bits down to 2^-29 of the row's largest value.
-__device__ inline int row_exponent(float mx) {
-  int e = 0;
-  frexpf(mx, &e);  // e = 0 for a zero row
-  return max(e, -100);
-}
-
-// The pre-split planes of one row's 4 normalised columns at quad q, scaled by
-// 2^(15 - e).
-__device__ inline void write_split_quad(const float (&v)[4], int e, int q, int64_t b, int cols, SplitPlanes sp) {
+// The pre-split planes of one row's 4 normalised columns at quad q (thread
+// = 4 consecutive columns; the threads of a 128-column chunk reduce its
+// maximum together, so every thread of the block must call this).
+__device__ inline void write_split_quad(const float (&v)[4], bool live, int q, int64_t b, int cols, SplitPlanes sp) {
   const int nchunks = (cols + kSplitChunk - 1) / kSplitChunk;
-  const float sc = ldexpf(1.0f, 15 - e);
+  const float mx = group_max<kSplitChunk / 4>(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+  if (!live) return;
+  int e2 = 0;
+  frexpf(mx, &e2);  // e2 = 0 for a zero chunk
+  e2 = max(e2, -100);
+  const float sc = ldexpf(1.0f, 15 - e2);
   uint16_t hi[4], lo[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float xs = v[i] * sc;
+  for (int e = 0; e < 4; ++e) {
+    const float xs = v[e] * sc;
     const _Float16 hh = static_cast<_Float16>(xs);
     const _Float16 ll = static_cast<_Float16>(xs - static_cast<float>(hh));
-    __builtin_memcpy(&hi[i], &hh, 2);
-    __builtin_memcpy(&lo[i], &ll, 2);
+    __builtin_memcpy(&hi[e], &hh, 2);
+    __builtin_memcpy(&lo[e], &ll, 2);
   }
   const int64_t off = b * cols + 4 * q;
   *reinterpret_cast<uint2*>(sp.hi + off) = make_uint2(hi[0] | (uint32_t{hi[1]} << 16), hi[2] | (uint32_t{hi[3]} << 16));
   *reinterpret_cast<uint2*>(sp.lo + off) = make_uint2(lo[0] | (uint32_t{lo[1]} << 16), lo[2] | (uint32_t{lo[3]} << 16));
-  if (q % (kSplitChunk / 4) == 0) sp.inv[b * nchunks + q / (kSplitChunk / 4)] = ldexpf(1.0f, e - 15);
+  if (q % (kSplitChunk / 4) == 0) sp.inv[b * nchunks + q / (kSplitChunk / 4)] = ldexpf(1.0f, e2 - 15);
 }
 
 // batch_residual_norm_kernel for a row of at most kResChunkQuads quads: every
@@ -464,7 +460,7 @@ template <bool kFinal, bool kSplit, int kResThreads>
 __device__ inline void residual_norm_row(float4* h4, const float4* p4, int64_t sstride, int splits, int nq, int cols,
                                          int b, const float* w, float eps, float* x, SplitPlanes sp,
                                          float4 (&red)[kResThreads / 256][kResChunkQuads],
-                                         float (&s_ss)[kResThreads / kWave], float (&s_mx)[kResThreads / kWave]) {
+                                         float (&s_ss)[kResThreads / kWave]) {
   constexpr int kResGroups = kResThreads / 256;
   const int grp = threadIdx.x / 256, t = threadIdx.x % 256;
   const int qq = min(t, nq - 1);
@@ -491,14 +487,6 @@ __device__ inline void residual_norm_row(float4* h4, const float4* p4, int64_t s
   float ss = live ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.0f;
   ss = group_sum<kWave>(ss);
   if (threadIdx.x % kWave == 0) s_ss[threadIdx.x / kWave] = ss;
-  if constexpr (kSplit) {
-    // max |h w|: times the scale, the row's largest |x| up to rounding (the
-    // exponent may come out one off at a power of two, which costs the planes
-    // nothing: their values stay below 2^16).
-    const float top = fmaxf(fmaxf(fabsf(v.x * wv.x), fabsf(v.y * wv.y)), fmaxf(fabsf(v.z * wv.z), fabsf(v.w * wv.w)));
-    const float mx = group_max<kWave>(live ? top : 0.0f);
-    if (threadIdx.x % kWave == 0) s_mx[threadIdx.x / kWave] = mx;
-  }
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
@@ -510,10 +498,10 @@ __device__ inline void residual_norm_row(float4* h4, const float4* p4, int64_t s
   for (int e = 0; e < 4; ++e) xv[e] = kFinal ? (hvv[e] * scale) * wvv[e] : hvv[e] * (scale * wvv[e]);
   if (x && live) *reinterpret_cast<float4*>(x + static_cast<int64_t>(b) * cols + 4 * t) = make_float4(xv[0], xv[1], xv[2], xv[3]);
   if constexpr (kSplit) {
-    float mx = 0.0f;
+    float sv[4];
 #pragma unroll
-    for (int i = 0; i < kResThreads / kWave; ++i) mx = fmaxf(mx, s_mx[i]);
-    if (live) write_split_quad(xv, row_exponent(mx * scale), t, b, cols, sp);
+    for (int e = 0; e < 4; ++e) sv[e] = live ? xv[e] : 0.0f;
+    write_split_quad(sv, live, t, b, cols, sp);
   }
 }
 
@@ -524,7 +512,7 @@ __global__ __launch_bounds__(kResThreads) void batch_residual_norm_kernel(float*
                                                                           L2WarmSet warm) {
   constexpr int kResGroups = kResThreads / 256;
   __shared__ float4 red[kResGroups][kResChunkQuads];
-  __shared__ float s_ss[kResThreads / kWave], s_mx[kResThreads / kWave];
+  __shared__ float s_ss[kResThreads / kWave];
   // Blocks past the rows: padding up to a multiple of kXcds, then the
   // L2-warming blocks (their loads land in red, 1 KB per wave).
   static_assert(sizeof(red) >= kResThreads / kWave * kWave * 16, "a 1 KB landing zone per wave");
@@ -541,7 +529,7 @@ __global__ __launch_bounds__(kResThreads) void batch_residual_norm_kernel(float*
   const float4* p4 = reinterpret_cast<const float4*>(part) + static_cast<int64_t>(b) * nq;
   const int64_t sstride = static_cast<int64_t>(batch) * nq;
   if (nq <= kResChunkQuads) {  // block-uniform
-    residual_norm_row<kFinal, kSplit, kResThreads>(h4, p4, sstride, splits, nq, cols, b, w, eps, x, sp, red, s_ss, s_mx);
+    residual_norm_row<kFinal, kSplit, kResThreads>(h4, p4, sstride, splits, nq, cols, b, w, eps, x, sp, red, s_ss);
     return;
   }
   float ss = 0.0f;
@@ -574,20 +562,40 @@ __global__ __launch_bounds__(kResThreads) void batch_residual_norm_kernel(float*
       xr[i] = kFinal ? (hr[i] * scale) * w[i] : hr[i] * (scale * w[i]);
   }
   if constexpr (kSplit) {
-    // The row's largest |x| first (s_ss was read above), then thread = 4
-    // consecutive columns.
-    auto value = [&](int i) { return kFinal ? (hr[i] * scale) * w[i] : hr[i] * (scale * w[i]); };
-    float mx = 0.0f;
-    for (int i = threadIdx.x; i < cols; i += kResThreads) mx = fmaxf(mx, fabsf(value(i)));
-    mx = group_max<kWave>(mx);
-    if (threadIdx.x % kWave == 0) s_mx[threadIdx.x / kWave] = mx;
-    __syncthreads();
+    // Thread = 4 consecutive columns; the threads of a chunk reduce its max
+    // together (whole chunks per pass), then write the planes.
+    const int nchunks = (cols + kSplitChunk - 1) / kSplitChunk;
+    for (int q0 = 0; q0 < nchunks * (kSplitChunk / 4); q0 += kResThreads) {  // block-uniform
+      const int q = q0 + static_cast<int>(threadIdx.x);
+      float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (4 * q < cols) {
 #pragma unroll
-    for (int i = 0; i < kResThreads / kWave; ++i) mx = fmaxf(mx, s_mx[i]);
-    const int e = row_exponent(mx);
-    for (int q = threadIdx.x; q < nq; q += kResThreads) {
-      const float v[4] = {value(4 * q), value(4 * q + 1), value(4 * q + 2), value(4 * q + 3)};
-      write_split_quad(v, e, q, b, cols, sp);
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * q + e;
+          v[e] = kFinal ? (hr[i] * scale) * w[i] : hr[i] * (scale * w[i]);
+        }
+      }
+      const float mx =
+          group_max<kSplitChunk / 4>(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+      if (4 * q < cols) {
+        int e2 = 0;
+        frexpf(mx, &e2);  // e2 = 0 for a zero chunk
+        e2 = max(e2, -100);
+        const float sc = ldexpf(1.0f, 15 - e2);
+        uint16_t hi[4], lo[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float xs = v[e] * sc;
+          const _Float16 hh = static_cast<_Float16>(xs);
+          const _Float16 ll = static_cast<_Float16>(xs - static_cast<float>(hh));
+          __builtin_memcpy(&hi[e], &hh, 2);
+          __builtin_memcpy(&lo[e], &ll, 2);
+        }
+        const int64_t off = static_cast<int64_t>(b) * cols + 4 * q;
+        *reinterpret_cast<uint2*>(sp.hi + off) = make_uint2(hi[0] | (uint32_t{hi[1]} << 16), hi[2] | (uint32_t{hi[3]} << 16));
+        *reinterpret_cast<uint2*>(sp.lo + off) = make_uint2(lo[0] | (uint32_t{lo[1]} << 16), lo[2] | (uint32_t{lo[3]} << 16));
+        if (q % (kSplitChunk / 4) == 0) sp.inv[static_cast<int64_t>(b) * nchunks + q / (kSplitChunk / 4)] = ldexpf(1.0f, e2 - 15);
+      }
     }
   }
 }

@@ -25,7 +25,7 @@ constexpr int kStageBytes = 2 * kPlaneBytes + kBN * kBK * 2;   // A hi, A lo, W
 constexpr int kActLd = kBN / 2 + 4;                            // floats per row of the act tile
 static_assert(kBM * kActLd * 4 <= kStages * kStageBytes, "act tile exceeds the stages");
 
-enum : int { kA32, kAPlanes };  // fp32 rows; fp16 planes with one scale per row
+enum : int { kA32, kAPlanes };  // fp32 rows; fp16 planes with one scale per row and 128 columns
 enum : int { kStore, kStoreSplit, kResidual, kSwiGlu };  // kStoreSplit: K split over gridDim.z
 
 // 16-byte chunk position of (row, chunk) in a stage [rows][8 chunks]: the 16
@@ -51,8 +51,9 @@ __device__ __forceinline__ int chunk_pos(int row, int chunk) { return row * kRow
 template <int kA, int kEpi>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_kernel(GemmArgs g) {
   __shared__ __align__(16) char lds[kStages * kStageBytes];
-  // fp32 A: the factor by which stage b's rows' sums change scale; at the end
-  // (and for planes) the rows' 1 / s.
+  // fp32 A: the factor by which stage b's rows' sums change scale, at the end
+  // the rows' 1 / s.  Planes: the 1 / s of the rows of a pair of stages (128
+  // columns), two pairs in turn.
   __shared__ __align__(16) float scale[kStages][kBM];
 
   const int tid = threadIdx.x, lane = tid % kWave;
@@ -81,6 +82,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     } else {
       g.a_hi += first * 2 * kBK;
       g.a_lo += first * 2 * kBK;
+      g.a_inv += first;
     }
     g.c += split * g.split_stride;
   }
@@ -97,11 +99,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int j = 0; j < kALoads; ++j) a_off[j] = kA == kA32 ? 0 : source(j, m0, g.m, g.lda);
 #pragma unroll
   for (int j = 0; j < kWLoads; ++j) w_off[j] = source(j, n0, g.n, g.k);
+  // Planes: waves 0 and 1 bring the scales of 64 rows each.
+  const uint32_t s_off = static_cast<uint32_t>(
+      min(m0 + wave * kWave + lane, g.m - 1) * static_cast<int64_t>(g.k / kSplitChunk) * 4);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
+  const uint32_t scale0 = __builtin_amdgcn_readfirstlane(lds_address(scale)) + wave * kWave * 4;
   auto issue = [&](int t, int buf) {
     const int64_t kb = static_cast<int64_t>(t) * kBK * 2;
     const uint32_t dst = lds0 + buf * kStageBytes + wave * 1024;
     if constexpr (kA != kA32) {
+      if (buf == 0 && wave < kBM / kWave)
+        dma_load<4>(g.a_inv + t / 2, s_off, scale0 + (t / 2) % 2 * (kBM * 4));
 #pragma unroll
       for (int j = 0; j < kALoads; ++j) {
         dma_load<16>(reinterpret_cast<const char*>(g.a_hi) + kb, a_off[j], dst + j * kWaves * 1024);
@@ -196,6 +204,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
   };
+  // Planes: the sums in `part`, each row's times its 1 / s.
+  auto flush_scaled = [&](const float* inv) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 sv = *reinterpret_cast<const float4*>(inv + wm * 64 + i * 32 + 8 * q + 4 * half);
+        const float s4[4] = {sv.x, sv.y, sv.z, sv.w};
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[i][j][4 * q + r] = fmaf(part[i][j][4 * q + r], s4[r], acc[i][j][4 * q + r]);
+      }
+  };
   // The sums of the rows times their factors.
   auto rescale = [&](const float* factors) {
 #pragma unroll
@@ -257,25 +280,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       if constexpr (kA == kA32) factor = scale[buf ^ 1][wm * 64 + lane];
       read(f0, buf ^ 1, 0);  // past the last stage: stale, not used
       multiply(f1, false);
-      if (last) flush();
+      if constexpr (kA == kA32) {
+        flush();
+      } else if (last) {
+        flush_scaled(&scale[t / 2 % 2][0]);
+      }
     };
     for (int t = 0; t < nk; t += 2) {
-      step(t, 0, true, kA == kA32);
+      step(t, 0, true, false);
       step(t + 1, 1, kA == kA32, true);
     }
   }
-  // The rows' 1 / s.
-  __syncthreads();
-  if constexpr (kA == kA32) {
+  if constexpr (kA == kA32) {  // the rows' 1 / s
+    __syncthreads();
     if (tid % 16 == 0) {
 #pragma unroll
       for (int u = 0; u < kPieces; ++u) scale[0][(tid + u * kThreads) / 16] = ldexpf(1.0f, e_run[u] - 15);
     }
-  } else if (tid < kBM) {
-    scale[0][tid] = g.a_inv[static_cast<int64_t>(min(m0 + tid, g.m - 1)) * (g.k / kSplitChunk)];
+    __syncthreads();
+    rescale(&scale[0][0]);
   }
-  __syncthreads();
-  rescale(&scale[0][0]);
 
   // Lane: column l32 of each 32 x 32 fragment, rows 8 q + 4 half + r.
   if constexpr (kEpi == kSwiGlu) {

@@ -282,9 +282,7 @@ hipError_t launch_qkv_postprocess(const QkvPostArgs& a, KvDtype kv, hipStream_t 
 // `chunk`-wide column chunk a power-of-two scale s (the chunk's max |a|
 // mapped into [2^14, 2^15)), hi = fp16(s a), lo = fp16(s a - hi), inv = 1 / s.
 // Written once by the kernel producing A, staged by every GEMM block.
-// kSplitChunk (one scale per GEMM K tile) is staged as is; its writer, the
-// residual + norm kernel, sees whole rows and gives every chunk of a row the
-// same scale, which the many-rows GEMM relies on.  kSplitChunkFine
+// kSplitChunk (one scale per GEMM K tile) is staged as is; kSplitChunkFine
 // suits producers that see 32 columns at a time (attention heads, the SwiGLU
 // epilogue) and is brought to one scale per K tile while staging.
 constexpr int kSplitChunk = 128;

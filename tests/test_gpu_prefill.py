@@ -412,3 +412,50 @@ def test_gemm_kernels_agree(gpu, monkeypatch):
     dma.synchronize()
     assert rel_err(dma.read_logits(), staged.read_logits()) < 1e-4
     assert dma.read_sequence(512, 1).tolist() == staged.read_sequence(512, 1).tolist()
+
+
+MM2_LAYER = dict(hidden_size=768, num_hidden_layers=1, num_attention_heads=8, num_key_value_heads=2, head_dim=96,
+                 intermediate_size=2048, vocab_size=6400, max_position_embeddings=32768, rms_norm_eps=1e-5,
+                 rope_theta=1e6, tie_word_embeddings=1)
+
+
+def layer_arrays(rng):
+    H, D, F = 768, 96, 2048
+    w = lambda rows, cols: f16_weights(rng, rows, cols)[1]  # noqa: E731
+    gain = lambda n: (1 + 0.1 * rng.standard_normal(n)).astype(np.float32)  # noqa: E731
+    return {"input_norm": gain(H), "post_attention_norm": gain(H), "q_norm": gain(D), "k_norm": gain(D),
+            "q_proj": w(8 * D, H), "k_proj": w(2 * D, H), "v_proj": w(2 * D, H), "o_proj": w(H, 8 * D),
+            "gate_proj": w(F, H), "up_proj": w(F, H), "down_proj": w(H, F)}
+
+
+def run_prefill_layer(mmr, arrays, hs, kv):
+    T, H = hs.shape
+    lw = mmr.LayerWeights.create(mmr.make_config(**MM2_LAYER), **arrays)
+    cache = mmr.KvCache(2, 96, T, kv)
+    x, y = mmr.DeviceArray.from_numpy(hs.reshape(-1)), mmr.DeviceArray(T * H, np.float32)
+    lw.prefill(cache, x, 0, T, y, mmr.DeviceArray(lw.prefill_workspace_size(T), np.uint8))
+    out = y.numpy().reshape(T, H), *cache.download(T)
+    lw.free()
+    return out
+
+
+@pytest.mark.parametrize("T", [512, 1500, 3000])
+def test_layer_planes_keep_small_channels_beside_a_large_gain(gpu, T):
+    # A channel whose gain is 2^30 times the others', in a chunk of 128 columns
+    # that no weight reads: the normalised rows' planes have one scale per 128
+    # columns, so every other chunk, and with them the layer's result and its
+    # cache rows, keep their bits.  512 rows: 64 x 64 tiles; 1,500: gate_up on
+    # the many-rows tiles and QKV on them in 3 K splits; 3,000: in 2.
+    mmr = gpu
+    print(f"[case] layer with a large gain T={T}", flush=True)
+    rng = np.random.default_rng(T)
+    arrays = layer_arrays(rng)
+    for n in ("q_proj", "k_proj", "v_proj", "gate_proj", "up_proj"):
+        arrays[n][:, 256:384] = 0.0
+    hs = rng.standard_normal((T, 768)).astype(np.float32)
+    want = run_prefill_layer(mmr, arrays, hs, mmr.KV_F32)
+    for n in ("input_norm", "post_attention_norm"):
+        arrays[n][300] *= np.float32(2.0**30)
+    got = run_prefill_layer(mmr, arrays, hs, mmr.KV_F32)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
