@@ -51,10 +51,12 @@ __device__ __forceinline__ int chunk_pos(int row, int chunk) { return row * kRow
 template <int kA, int kEpi>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_kernel(GemmArgs g) {
   __shared__ __align__(16) char lds[kStages * kStageBytes];
-  // fp32 A: the factor by which stage b's rows' sums change scale, at the end
-  // the rows' 1 / s.  Planes: the 1 / s of the rows of a pair of stages (128
-  // columns), two pairs in turn.
-  __shared__ __align__(16) float scale[kStages][kBM];
+  // The rows' 1 / s.  Planes: of a pair of stages (128 columns), two pairs in
+  // turn.  fp32 A: of a stage's kScaleCols columns each, four stages in turn (a
+  // wave may be staging t + 2 while another still adds up t).
+  constexpr int kScaleCols = kEpi == kStoreSplit ? kSplitChunkFine : kBK;
+  constexpr int kStageScales = kA == kA32 ? kBK / kScaleCols : 1;
+  __shared__ __align__(16) float scale[kA == kA32 ? 4 * kStageScales : 2][kBM];
 
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -122,26 +124,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   };
 
   // fp32 A: this thread's four 4-column pieces of a stage, row (tid + 512 u)
-  // / 16, columns 4 (tid % 16).  The 16 lanes of a row find its maximum
-  // together; the row's scale s = 2^(15 - e) follows the largest |a| seen so
-  // far, and the sums so far follow the scale (a power of two, exact).
-  constexpr int kPieces = kBM * kBK / 4 / kThreads;
+  // / 16, columns 4 (tid % 16).  The lanes of a row's kScaleCols columns find
+  // their maximum together, and with it the scale s = 2^(15 - e).
+  constexpr int kPieces = kBM * kBK / 4 / kThreads, kPieceRows = kThreads / 16;
+  const int a_row = tid / 16, a_col = tid % 16;
   float4 areg[kA == kA32 ? kPieces : 1];
-  int e_run[kA == kA32 ? kPieces : 1];
-  auto load_a = [&](int t) {
+  const float* a_rows = kA == kA32 ? g.a + static_cast<int64_t>(m0) * g.lda : nullptr;
+  uint32_t a_src[kPieces];  // bytes from there: under 128 rows of lda < 2^23
 #pragma unroll
-    for (int u = 0; u < kPieces; ++u) {
-      const int row = min(m0 + (tid + u * kThreads) / 16, g.m - 1);
-      areg[u] = *reinterpret_cast<const float4*>(g.a + static_cast<int64_t>(row) * g.lda + t * kBK + tid % 16 * 4);
-    }
+  for (int u = 0; u < kPieces; ++u)
+    a_src[u] = static_cast<uint32_t>(min(a_row + u * kPieceRows, g.m - 1 - m0) * (g.lda * int64_t{4}) + a_col * 16);
+  auto load_a = [&](int t) {
+    const char* base = reinterpret_cast<const char*>(a_rows + t * kBK);
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) areg[u] = *reinterpret_cast<const float4*>(base + a_src[u]);
   };
-  auto store_a = [&](int buf, int u0, int u1) {
+  // Rows 32 on, a piece's chunk keeps its place in the row.
+  static_assert(kPieceRows % 16 == 0, "chunk_pos repeats every 16 rows");
+  char* const a_dst = lds + chunk_pos(a_row, a_col / 2) * 16 + a_col % 2 * 8;
+  float* const s_dst = &scale[a_col / (kScaleCols / 4)][a_row];
+  auto store_a = [&](int t, int buf, int u0, int u1) {
 #pragma unroll
     for (int u = u0; u < u1; ++u) {
-      const int row = (tid + u * kThreads) / 16, q = tid % 16;
       const float4 v = areg[u];
-      const float mx = group_max<16>(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-      const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx), e_run[u]) : e_run[u];
+      const float mx = group_max<kScaleCols / 4>(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+      const int e = max(__builtin_amdgcn_frexp_expf(mx), -100);  // 0 for a zero chunk
       const float sc = ldexpf(1.0f, 15 - e);
       const float x[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
       f16x4 hi, lo;
@@ -150,11 +157,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         hi[j] = static_cast<_Float16>(x[j]);
         lo[j] = static_cast<_Float16>(x[j] - static_cast<float>(hi[j]));
       }
-      char* dst = lds + buf * kStageBytes + chunk_pos(row, q / 2) * 16 + q % 2 * 8;
+      char* dst = a_dst + buf * kStageBytes + u * kPieceRows * kRowChunks * 16;
       *reinterpret_cast<f16x4*>(dst) = hi;
       *reinterpret_cast<f16x4*>(dst + kPlaneBytes) = lo;
-      if (q == 0) scale[buf][row] = ldexpf(1.0f, e_run[u] - e);
-      e_run[u] = e;
+      // The lanes of a group write the same value to the same place.
+      s_dst[t % 4 * kStageScales * kBM + u * kPieceRows] = ldexpf(1.0f, e - 15);
     }
   };
 
@@ -184,9 +191,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int j = 0; j < 2; ++j) f.w[j] = *reinterpret_cast<const f16x8*>(st + w_rd[ks] + j * 4096);
   };
-  // Sums run in two levels: the products of kSplitChunk columns (one stage of
-  // fp32 A) in `part`, then into `acc`; a single chain of K / 16 additions
-  // doubled the error against 64 bits.
+  // Sums run in two levels: the products of the columns under one scale in
+  // `part`, then, each row's times its 1 / s, into `acc`; a single chain of K / 16
+  // additions doubled the error against 64 bits.
   auto multiply = [&](const Frags& f, bool fresh) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -198,14 +205,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int j = 0; j < 2; ++j) part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.w[j], part[i][j], 0, 0, 0);
   };
-  auto flush = [&] {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
-  };
-  // Planes: the sums in `part`, each row's times its 1 / s.
-  auto flush_scaled = [&](const float* inv) {
+  auto flush = [&](const float* inv) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -218,20 +218,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
           for (int r = 0; r < 4; ++r)
             acc[i][j][4 * q + r] = fmaf(part[i][j][4 * q + r], s4[r], acc[i][j][4 * q + r]);
       }
-  };
-  // The sums of the rows times their factors.
-  auto rescale = [&](const float* factors) {
+    if constexpr (kA == kA32) {
+      // Here, and not sunk to the next use of acc past store_a's branch: both
+      // sums and the next products' would be live at once and spill.
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 sv = *reinterpret_cast<const float4*>(factors + wm * 64 + i * 32 + 8 * q + 4 * half);
-        const float s4[4] = {sv.x, sv.y, sv.z, sv.w};
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] *= s4[r];
-      }
+        for (int j = 0; j < 2; ++j) asm volatile("" : "+v"(acc[i][j]));
+    }
   };
 
   // Each k step's fragments are read while the one before is multiplied,
@@ -241,10 +235,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   {
     issue(0, 0);
     if constexpr (kA == kA32) {
-#pragma unroll
-      for (int u = 0; u < kPieces; ++u) e_run[u] = -100;
       load_a(0);
-      store_a(0, 0, kPieces);
+      store_a(0, 0, 0, kPieces);
     }
     issue(1, 1);
     if constexpr (kA == kA32) load_a(1);
@@ -255,50 +247,34 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                  : "memory");
     Frags f0, f1;
     read(f0, 0, 0);
-    float factor = 1.0f;
+    constexpr bool kHalves = kA == kA32 && kStageScales == 2;  // a scale per two k steps
     auto step = [&](int t, int buf, bool fresh, bool last) {
-      if constexpr (kA == kA32) {
-        if (__any(factor != 1.0f)) rescale(&scale[buf][0]);
-      }
       read(f1, buf, 1);
       multiply(f0, fresh);
       if constexpr (kA == kA32) {
-        if (t + 1 < nk) store_a(buf ^ 1, 0, kPieces / 2);
+        if (t + 1 < nk) store_a(t + 1, buf ^ 1, 0, kPieces / 2);
       }
       read(f0, buf, 2);
       multiply(f1, false);
+      if constexpr (kHalves) flush(&scale[t % 4 * kStageScales][0]);
       if constexpr (kA == kA32) {
-        if (t + 1 < nk) store_a(buf ^ 1, kPieces / 2, kPieces);
+        if (t + 1 < nk) store_a(t + 1, buf ^ 1, kPieces / 2, kPieces);
       }
       read(f1, buf, 3);
-      multiply(f0, false);
+      multiply(f0, kHalves);
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       if (t + 2 < nk) {
         issue(t + 2, buf);
         if constexpr (kA == kA32) load_a(t + 2);
       }
-      if constexpr (kA == kA32) factor = scale[buf ^ 1][wm * 64 + lane];
       read(f0, buf ^ 1, 0);  // past the last stage: stale, not used
       multiply(f1, false);
-      if constexpr (kA == kA32) {
-        flush();
-      } else if (last) {
-        flush_scaled(&scale[t / 2 % 2][0]);
-      }
+      if (last) flush(&scale[kA == kA32 ? t % 4 * kStageScales + kStageScales - 1 : t / 2 % 2][0]);
     };
     for (int t = 0; t < nk; t += 2) {
-      step(t, 0, true, false);
+      step(t, 0, true, kA == kA32);
       step(t + 1, 1, kA == kA32, true);
     }
-  }
-  if constexpr (kA == kA32) {  // the rows' 1 / s
-    __syncthreads();
-    if (tid % 16 == 0) {
-#pragma unroll
-      for (int u = 0; u < kPieces; ++u) scale[0][(tid + u * kThreads) / 16] = ldexpf(1.0f, e_run[u] - 15);
-    }
-    __syncthreads();
-    rescale(&scale[0][0]);
   }
 
   // Lane: column l32 of each 32 x 32 fragment, rows 8 q + 4 half + r.
@@ -453,7 +429,7 @@ bool gemm_many_rows(const GemmArgs& g) {
          (!g.a_hi || g.a_chunk == kSplitChunk) && (!g.swiglu || (g.n % 8 == 0 && g.ldc % 4 == 0)) &&
          (reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.a_hi) | reinterpret_cast<uintptr_t>(g.a_lo) |
           reinterpret_cast<uintptr_t>(g.w)) % 16 == 0 &&
-         a_bytes < (int64_t{1} << 32) && w_bytes < (int64_t{1} << 32);
+         a_bytes < (int64_t{1} << 32) && w_bytes < (int64_t{1} << 32) && g.lda < (1 << 23);
 }
 
 hipError_t launch_gemm_many_rows(const GemmArgs& g, hipStream_t stream) {

@@ -83,6 +83,26 @@ def test_matmul_many_rows_matches_fp64(gpu, batch, rows, cols, grow):
         assert rel_err(dr.numpy(), res + exact) < 1e-5
 
 
+@pytest.mark.parametrize("batch,rows,cols", [(100, 1152, 768), (1536, 2048, 768), (70, 24576, 384)])
+def test_matmul_keeps_small_columns_beside_large_ones(gpu, batch, rows, cols):
+    # columns 2^30 times the others' size in a chunk of 128 that no weight
+    # reads: x is split under a scale per 128 columns or fewer, so the result
+    # keeps its bits (the 64 x 64 tiles, then the many-rows ones)
+    mmr = gpu
+    print(f"[case] matmul beside large columns {batch}x{rows}x{cols}", flush=True)
+    rng = np.random.default_rng(batch)
+    w16, _ = f16_weights(rng, rows, cols)
+    w16[:, 128:256] = 0
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    dw, dy = mmr.DeviceArray.from_numpy(w16.view(np.uint16)), mmr.DeviceArray((batch, rows), np.float32)
+    out = []
+    for size in (1.0, 2.0**30):
+        x[:, 128:256] *= np.float32(size)
+        mmr.matmul_f16(dw, rows, cols, mmr.DeviceArray.from_numpy(x), batch, dy)
+        out.append(dy.numpy())
+    np.testing.assert_array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("batch", [16, 17, 32, 33, 64, 65])
 def test_matmul_few_rows_wide_output_matches_fp64(gpu, batch):
     # 160 tiles of 128 x 256 with few of their rows: the edges between the
@@ -457,5 +477,25 @@ def test_layer_planes_keep_small_channels_beside_a_large_gain(gpu, T):
     for n in ("input_norm", "post_attention_norm"):
         arrays[n][300] *= np.float32(2.0**30)
     got = run_prefill_layer(mmr, arrays, hs, mmr.KV_F32)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("T", [512, 1500, 3000])
+def test_layer_act_keeps_small_columns_beside_large_ones(gpu, T):
+    # 32 FFN columns 2^18 times the others' size that the down projection does
+    # not read: act is split under a scale per 32 columns, pre-split (512 and
+    # 1,500 rows) and in the many-rows GEMM's K splits (3,000)
+    mmr = gpu
+    print(f"[case] layer with large FFN columns T={T}", flush=True)
+    rng = np.random.default_rng(T)
+    arrays = layer_arrays(rng)
+    arrays["up_proj"][1056:1088] *= np.float32(2.0**-9)  # exact in fp16 on both sides
+    arrays["up_proj"] = arrays["up_proj"].astype(np.float16).astype(np.float32)
+    arrays["down_proj"][:, 1056:1088] = 0.0
+    hs = rng.standard_normal((T, 768)).astype(np.float32)
+    want = run_prefill_layer(mmr, arrays, hs, mmr.KV_F16)
+    arrays["up_proj"][1056:1088] *= np.float32(2.0**27)
+    got = run_prefill_layer(mmr, arrays, hs, mmr.KV_F16)
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g, w)
