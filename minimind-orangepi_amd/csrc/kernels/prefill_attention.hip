@@ -440,21 +440,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // x 4 query heads of one KV group, its 8 waves 4 heads x 2 key ranges.  K, V,
 // q and p all go to the matrix cores as hi + lo fp16 planes (22 bits; the lo x
 // lo products, 2^-22 of the others, are left out), with power-of-two scales
-// that keep every plane below 2^15: q per query, K and V per 8 keys, which are
-// the rows one wave stages and four of a lane's 16 scores, and p per 8 keys so
-// that O^T keeps one scale 2^(30 - E), E the largest V exponent so far.  K and
-// V pass through registers, where they are split, into the stage that the four
-// heads share.
+// that keep every plane below 2^15: q per query; K per 8 keys, four of a lane's
+// 16 scores; V per tile of 32 keys and D / 4 dims, whose products are summed
+// before they meet O^T, so that O^T has no scale; p a fixed 2^15.  A value
+// keeps the 22 bits down to 2^-17 of the largest under its scale, below that
+// 2^-40 of the largest.  K and V pass through registers, where they are split,
+// into the stage that the four heads share: a wave stages 8 rows of K and D / 4
+// dims of all 32 rows of V, so that each scale is its own to find.
 //
-// What bounds it: the matrix cores, 36 products of 32 cycles a tile and head
-// for d = 96 (1,152 cycles, where products of fp32 operands would take 6,144),
-// and the splits' and the softmax's vector instructions beside them.
-// prefill.hip's kernel / this one, 8 query heads on 2: d 96, 2,000 rows 118.9
-// / 88.5 us, 4,096 rows 398.5 / 171.1, 3,000 rows after 1,111 keys 349.9 /
-// 171.5; d 64 78.6 / 70.6, 249.6 / 136.9, 221.5 / 137.2.  Largest error
-// against 64 bits, of the largest value: d 96, 4,096 rows 3.5e-7 / 2.6e-7,
-// 3,000 rows after 3,000 keys 5.6e-7 / 3.4e-7 (a tile's values are summed
-// before they meet the long sums; added product by product it was 5.9e-7).
+// What bounds it: 36 products of 32 cycles a tile and head for d = 96 (1,152
+// cycles, where products of fp32 operands would take 6,144), and the splits' and
+// the softmax's vector instructions beside them.  prefill.hip's kernel / this
+// one, 8 query heads on 2: d 96, 2,000 rows 118.9 / 90.6 us, 4,096 rows 398.1 /
+// 173.2, 3,000 rows after 1,111 keys 349.8 / 174.6; d 64 77.6 / 71.5, 248.3 /
+// 136.5, 222.4 / 137.6.  Error against 64 bits of each dimension, of its own
+// largest value (d 96, 2,000 rows after 2,000 keys): 2.0e-6 / 1.1e-6; with V's
+// dimensions spread over 2^16 1.9e-6 / 1.1e-6, its keys over 2^20 2.2e-6 /
+// 1.8e-6, q and (inversely) k over 2^8 1.9e-6 / 1.2e-6.  (A tile's values are
+// summed before they meet the long sums: added product by product, 3,000 rows
+// after 3,000 keys had 5.9e-7 of the largest value against 3.4e-7.  Under one V
+// scale per 8 keys and all dims, dimensions 2^-20 of the others' size had 8.7e-6
+// of their own; they still do where they share their D / 4 with large ones.
+// Scales per 8 dims: 173 -> 198 us, for their maxima over the wave; per 32 dims
+// and 8 rows a wave, exchanged through LDS: 195 us.)
 constexpr int kHeads32 = 4;
 template <int D, bool kPool>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attention_f32_kernel(
@@ -467,10 +475,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   constexpr int kStages = 2 * S * kStageBytes;
   constexpr int kLdsBytes = kStages > kMergeFloats * 4 * kWaves / 2 ? kStages : kMergeFloats * 4 * kWaves / 2;
   constexpr int DJ = D / 16, DT = D / 32;
+  constexpr int C = D / HB;           // dims of V under one scale
   constexpr int kPer = D / 32;        // float4s of K (and of V) that a thread stages per tile
-  constexpr int kMinScoreExp = -40;  // smaller q or k count as 2^-40: their scores are 0 to fp32
+  // Rows of q and k are scaled as at least 2^-40, so that a masked score's -inf
+  // never meets a factor of 0; below 2^-57 they keep fewer than 22 bits.
+  constexpr int kMinScoreExp = -40;
+  constexpr int kMinValueExp = -100;
   __shared__ __align__(16) char lds[kLdsBytes];
-  __shared__ __align__(16) int k_exp[2][S][4], v_exp[2][S][4];
+  __shared__ __align__(16) int k_exp[2][S][HB], v_exp[2][S][HB];
 
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -485,17 +497,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const int n_tiles = last_key / kKeyTile + 1;
   const int n_iter = (n_tiles + S - 1) / S;
 
-  // This wave stages rows 8 hb .. + 7 of a tile: float4 lane + 64 i of them.
-  int srow[kPer], scol[kPer], spos[kPer];
+  // This wave stages rows 8 hb .. + 7 of a K tile, eight lanes a row, and dims
+  // C hb .. + C - 1 of a V tile's 32 rows.
+  static_assert(8 * HB == kKeyTile && kPer * kWave * 4 == kKeyTile * C, "tile split over the waves");
+  const int krow = 8 * hb + lane / 8;
+  auto vrow = [&](int u) { return (lane + u * kWave) / (C / 4); };
+  int koff[kPer], kpos[kPer], voff[kPer], vpos[kPer];  // elements from the tile in memory, bytes from its plane
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int f = lane + i * kWave;
-    srow[i] = 8 * hb + f / (D / 4);
-    scol[i] = f % (D / 4) * 4;
-    spos[i] = tile_chunk<D>(srow[i], scol[i] / 8) * 16 + scol[i] % 8 * 2;
+  for (int u = 0; u < kPer; ++u) {
+    const int kcol = 32 * u + lane % 8 * 4, vcol = C * hb + (lane + u * kWave) % (C / 4) * 4;
+    koff[u] = krow * D + kcol;
+    kpos[u] = tile_chunk<D>(krow, kcol / 8) * 16 + kcol % 8 * 2;
+    voff[u] = vrow(u) * D + vcol;
+    vpos[u] = tile_chunk<D>(vrow(u), vcol / 8) * 16 + vcol % 8 * 2;
   }
   f32x4 kreg[kPer], vreg[kPer];
-  auto load = [&](f32x4 (&r)[kPer], void* const* seg_base, const void* pool, int i) {
+  auto load = [&](f32x4 (&r)[kPer], const int (&whole)[kPer], auto row, void* const* seg_base, const void* pool, int i) {
     const int t0 = min(s + i * S, n_tiles - 1) * kKeyTile;
     const float* base;
     if constexpr (kPool) {
@@ -506,19 +523,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     }
     const int limit = last_key - t0;  // rows past the last key are masked, any key's row will do
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) r[u] = *reinterpret_cast<const f32x4*>(base + min(srow[u], limit) * D + scol[u]);
+    for (int u = 0; u < kPer; ++u) {
+      uint32_t off = whole[u];
+      if (limit < kKeyTile - 1) off -= static_cast<uint32_t>(max(row(u) - limit, 0) * D);  // wave-uniform branch
+      r[u] = *reinterpret_cast<const f32x4*>(base + off);
+    }
   };
   static_assert(sizeof(KvSeg) == 2 * sizeof(void*), "segments are (k, v) pairs");
-  auto load_k = [&](int i) { load(kreg, &a.seg.s[0].k, a.pool.k, i); };
-  auto load_v = [&](int i) { load(vreg, &a.seg.s[0].v, a.pool.v, i); };
+  auto load_k = [&](int i) { load(kreg, koff, [&](int) { return krow; }, &a.seg.s[0].k, a.pool.k, i); };
+  auto load_v = [&](int i) { load(vreg, voff, vrow, &a.seg.s[0].v, a.pool.v, i); };
   char* stage0 = lds + s * kStageBytes;
   auto stage = [&](int parity) { return stage0 + parity * S * kStageBytes; };
-  // The wave's 8 rows to one exponent (at least `least`) and two planes.
-  auto store = [&](const f32x4 (&r)[kPer], char* hi_plane, int* exponent, int least) {
+  static_assert(C % 8 == 0, "a scale for whole runs of 8 dims");
+  auto largest = [](const f32x4& r) {
+    return fmaxf(fmaxf(fabsf(r[0]), fabsf(r[1])), fmaxf(fabsf(r[2]), fabsf(r[3])));
+  };
+  // The wave's share of a tile to one exponent (at least `least`) and two planes.
+  auto store = [&](const f32x4 (&r)[kPer], const int (&pos)[kPer], char* hi_plane, int* exponent, int least) {
     float mx = 0.0f;
 #pragma unroll
-    for (int u = 0; u < kPer; ++u)
-      mx = fmaxf(fmaxf(fmaxf(mx, fabsf(r[u][0])), fmaxf(fabsf(r[u][1]), fabsf(r[u][2]))), fabsf(r[u][3]));
+    for (int u = 0; u < kPer; ++u) mx = fmaxf(mx, largest(r[u]));
     mx = group_max<kWave>(mx);
     const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx), least) : least;
     const float sc = ldexpf(1.0f, 15 - e);
@@ -527,13 +551,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
       uint32_t hw[2], lw[2];
 #pragma unroll
       for (int w = 0; w < 2; ++w) split2(r[u][2 * w] * sc, r[u][2 * w + 1] * sc, hw[w], lw[w]);
-      *reinterpret_cast<uint2*>(hi_plane + spos[u]) = make_uint2(hw[0], hw[1]);
-      *reinterpret_cast<uint2*>(hi_plane + kPlaneBytes + spos[u]) = make_uint2(lw[0], lw[1]);
+      *reinterpret_cast<uint2*>(hi_plane + pos[u]) = make_uint2(hw[0], hw[1]);
+      *reinterpret_cast<uint2*>(hi_plane + kPlaneBytes + pos[u]) = make_uint2(lw[0], lw[1]);
     }
     if (lane == 0) exponent[hb] = e;
   };
-  auto store_k = [&](int parity) { store(kreg, stage(parity), k_exp[parity][s], kMinScoreExp); };
-  auto store_v = [&](int parity) { store(vreg, stage(parity) + 2 * kPlaneBytes, v_exp[parity][s], -100); };
+  auto store_k = [&](int parity) { store(kreg, kpos, stage(parity), k_exp[parity][s], kMinScoreExp); };
+  auto store_v = [&](int parity) { store(vreg, vpos, stage(parity) + 2 * kPlaneBytes, v_exp[parity][s], kMinValueExp); };
   auto barrier = [&] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
   load_k(0);
@@ -571,11 +595,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     }
   }
 
-  f32x16 ot[DT];  // O^T 2^(30 - e_run): [dim 32 jt + 8 (i / 4) + 4 half + i % 4][query qi]
+  f32x16 ot[DT];  // O^T[dim 32 jt + 8 (i / 4) + 4 half + i % 4][query qi]
 #pragma unroll
   for (int j = 0; j < DT; ++j) ot[j] = f32x16{};
   float m_run = -INFINITY, l_part = 0.0f, alpha = 1.0f;
-  int e_run = -100;
+  float v_unit[HB];  // 2^(e - 30) of the V tile whose values come next, e its exponents
+#pragma unroll
+  for (int j = 0; j < HB; ++j) v_unit[j] = 0.0f;
   bool grew = false;  // wave-uniform
 
   auto scores = [&](int parity) {
@@ -597,7 +623,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const char* vst = stage(parity) + 2 * kPlaneBytes + lane % 2 * 8;
 #pragma unroll
     for (int jt = 0; jt < DT; ++jt) {
-      f32x16 sum{};  // the tile's, before O^T's: a sixth of the roundings at O^T's size
+      f32x16 sum{};  // the tile's, 2^(30 - e) times: a sixth of the roundings at O^T's size
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int row = 16 * t + 4 * half + lane % 16 / 4;
@@ -615,7 +641,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[t], sum, 0, 0, 0);
         sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[t], sum, 0, 0, 0);
       }
-      ot[jt] += sum;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ot[jt][e] = fmaf(sum[e], v_unit[(32 * jt + 8 * (e / 4)) / C], ot[jt][e]);
     }
   };
 
@@ -650,8 +677,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     for (int q = 0; q < 4; ++q)
       mx = fmaxf(mx, fmaxf(fmaxf(st[4 * q], st[4 * q + 1]), fmaxf(st[4 * q + 2], st[4 * q + 3])) * inv[q]);
     mx = half_swap_max(mx);
-    // Tile i - 1's rise of the maximum or of V's exponent reaches O^T before
-    // its values do.
+    // Tile i - 1's rise of the maximum reaches O^T before its values do.
     if (grew) {
 #pragma unroll
       for (int j = 0; j < DT; ++j) ot[j] *= alpha;
@@ -669,18 +695,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     kx = *reinterpret_cast<const int4*>(&k_exp[kParity ^ 1][s][0]);
     if (i > 0) add_pv(kParity ^ 1);
     const int4 vx = *reinterpret_cast<const int4*>(&v_exp[kParity][s][0]);
-    const int e_new = max(max(e_run, max(vx.x, vx.y)), max(vx.z, vx.w));
-    grew = grew || e_new != e_run;
-    alpha = ldexpf(alpha, e_run - e_new);
-    e_run = e_new;
-    const float cg[4] = {ldexpf(1.0f, 15 + vx.x - e_new), ldexpf(1.0f, 15 + vx.y - e_new),
-                         ldexpf(1.0f, 15 + vx.z - e_new), ldexpf(1.0f, 15 + vx.w - e_new)};
+    const int ve[HB] = {vx.x, vx.y, vx.z, vx.w};
+#pragma unroll
+    for (int j = 0; j < HB; ++j) v_unit[j] = ldexpf(1.0f, __builtin_amdgcn_readfirstlane(ve[j]) - 30);
     float p[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(st[e], inv[e / 4], -m_use));
     l_part += sum16(p);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) p[e] *= cg[e / 4];
+    for (int e = 0; e < 16; ++e) p[e] *= 32768.0f;
 #pragma unroll
     for (int t = 0; t < 2; ++t) split8(p + 8 * t, ph[t], pl[t]);
     st = st_next;
@@ -697,9 +720,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     for (int j = 0; j < DT; ++j) ot[j] *= alpha;
   }
   add_pv((n_iter - 1) & 1);
-  const float unit = ldexpf(1.0f, e_run - 30);
-#pragma unroll
-  for (int j = 0; j < DT; ++j) ot[j] *= unit;
   merge_and_write<D, HB>(a, ot, m_run, l_part, reinterpret_cast<float*>(lds), s, hb, lane, h, b, q0);
 }
 

@@ -280,6 +280,47 @@ def test_prefill_attention_many_rows_f32(gpu, d, hq, hkv, start, T, spread):
         assert err.max() < 2e-6, (h, int(err.argmax()), float(err.max()))
 
 
+@pytest.mark.parametrize("d", [64, 96])
+@pytest.mark.parametrize("hq,hkv,start,T", [(16, 4, 0, 993), (8, 2, 1990, 2000)])
+def test_prefill_attention_f32_keeps_small_dims(gpu, d, hq, hkv, start, T):
+    # V's dims have a scale of their own, per run of d / 4: dims 2^-40 of the
+    # others' size come out as the same bits, 2^-40 times; and with dims spread
+    # over 2^16 and, in the other half, keys over 2^16, every dim is within 5e-6
+    # of its own largest value (22 bits of K, V, q and p; a score of size 10
+    # turns two of these into 3.4e-6 of p at most).
+    mmr = gpu
+    print(f"[case] prefill attention f32 small dims d={d} hq={hq} hkv={hkv} start={start} T={T}", flush=True)
+    rng = np.random.default_rng(d + hq + start)
+    n = start + T
+    k = rng.standard_normal((hkv, n, d)).astype(np.float32)
+    v = rng.standard_normal((hkv, n, d)).astype(np.float32)
+    q = rng.standard_normal((T, hq, d)).astype(np.float32)
+    dq, out = mmr.DeviceArray.from_numpy(q.reshape(T, hq * d)), mmr.DeviceArray((T, hq * d), np.float32)
+
+    def attend(v):
+        cache = mmr.KvCache(hkv, d, n, mmr.KV_F32)
+        cache.upload(k, v)
+        mmr.prefill_attention(dq, cache, start, T, hq, hkv, d, out)
+        return out.numpy().reshape(T, hq, d)
+
+    size = np.ones(d, np.float32)
+    size[d // 4: d // 2] = 2.0**-40
+    np.testing.assert_array_equal(attend(v * size), attend(v) * size)
+
+    v[:, :, : d // 2] *= np.exp2(rng.uniform(-16, 0, (hkv, 1, d // 2))).astype(np.float32)
+    v[:, :, d // 2:] *= np.exp2(rng.uniform(-16, 0, (hkv, n, 1))).astype(np.float32)
+    got = attend(v)
+    hidden = np.arange(n)[None, :] > start + np.arange(T)[:, None]
+    for h in range(hq):
+        g = h // (hq // hkv)
+        s = q[:, h].astype(np.float64) @ k[g].astype(np.float64).T / np.sqrt(d)
+        s[hidden] = -np.inf
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        ref = p @ v[g].astype(np.float64) / p.sum(axis=1, keepdims=True)
+        err = np.abs(got[:, h] - ref).max(axis=0) / np.abs(ref).max(axis=0)
+        assert err.max() < 5e-6, (h, int(err.argmax()), float(err.max()))
+
+
 def synth_model(mmr, g):
     return mmr.Model.synthetic(mmr.make_config(**g["config"]), g["seed"], g["std"], g["round_fp16"])
 
