@@ -82,7 +82,7 @@ __device__ __forceinline__ float sum16(const float (&p)[16]) {
 
 // The end of a block: the key ranges' (m, l) per query and O^T, as the lanes
 // of wave (s, hb) hold them, merge pairwise through `mrg`, and range 0's waves
-// write the rows.
+// write the rows.  The block has met since `mrg` was last read.
 template <int D, int HB>
 __device__ __forceinline__ void merge_and_write(const PrefillAttnArgs& a, f32x16 (&ot)[D / 32], float m_run,
                                                 float l_part, float* mrg, int s, int hb, int lane, int h, int b,
@@ -92,7 +92,7 @@ __device__ __forceinline__ void merge_and_write(const PrefillAttnArgs& a, f32x16
   const int qi = lane % 32, half = lane / 32;
 #pragma unroll
   for (int step = S / 2; step >= 1; step /= 2) {
-    __syncthreads();  // the stages (or the previous round's values) have been read
+    if (step < S / 2) __syncthreads();  // the previous round's values have been read
     if (s >= step && s < 2 * step) {
       float* dst = mrg + ((s - step) * HB + hb) * kMergeFloats;
 #pragma unroll
@@ -168,6 +168,100 @@ __device__ __forceinline__ void merge_and_write(const PrefillAttnArgs& a, f32x16
   }
 }
 
+// Whether any wave of the block holds an infinity or a NaN (`bad` is LDS of its
+// own; the waves meet here).
+template <int DT>
+__device__ __forceinline__ bool block_not_finite(const f32x16 (&ot)[DT], float l_part, int (&bad)[kWaves], int wave,
+                                                 int lane) {
+  float z = l_part * 0.0f;
+#pragma unroll
+  for (int j = 0; j < DT; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z = fmaf(ot[j][i], 0.0f, z);
+  const bool mine = __any(z != 0.0f);
+  if (lane == 0) bad[wave] = mine;
+  __syncthreads();
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) any |= bad[w];
+  return __builtin_amdgcn_readfirstlane(any) != 0;
+}
+
+// The block's rows once more, in plain fp32 and over each query's own keys
+// only.  An infinite or NaN key or value reaches, on the matrix cores, every
+// query of its tile (0 times it is NaN, also where the key is masked), and with
+// split operands every value under its scale.  Here it reaches what the formula
+// says: scores of -inf count for nothing, a value touches its own dim, and
+// queries before it stay as they are.  Wave: HB heads x queries s, s + S, ...;
+// lane: a key of 64 for the scores, dims lane and lane + 64 for the values.
+template <typename KV, int D, int HB, bool kPool>
+__device__ void attend_rows_plainly(const PrefillAttnArgs& a, int s, int lane, int h, int b, int q0) {
+  constexpr int S = kWaves / HB;
+  static_assert(D <= 2 * kWave && kKvPage == kWave, "two dims a lane, a page of keys a step");
+  const int g = h / (a.hq / a.hkv);
+  const float qscale = 1.4426950408889634f / sqrtf(static_cast<float>(D));
+  const int rows = min(kQueryTile, a.tokens - q0);
+  for (int qi = s; qi < rows; qi += S) {
+    const int qpos = a.start + q0 + qi;
+    const int64_t row = static_cast<int64_t>(b) * a.tokens + q0 + qi;
+    const float* q = a.query + row * a.query_stride + h * D;
+    float m_run = -INFINITY, l = 0.0f, o[2] = {0.0f, 0.0f};
+    for (int t0 = 0; t0 <= qpos; t0 += kWave) {
+      const KV *k, *v;
+      if constexpr (kPool) {
+        const int64_t off = kv_pool_offset(a.pool.interleave, b, t0, g, a.hkv, D);
+        k = static_cast<const KV*>(a.pool.k) + off;
+        v = static_cast<const KV*>(a.pool.v) + off;
+      } else {
+        const int seg = kv_segment(t0);
+        const int64_t off = kv_segment_offset(seg, t0, g, a.hkv, D);
+        k = static_cast<const KV*>(a.seg.s[seg].k) + off;
+        v = static_cast<const KV*>(a.seg.s[seg].v) + off;
+      }
+      const int keys = min(kWave, qpos + 1 - t0);
+      const KV* key = k + min(lane, keys - 1) * D;
+      float dot = 0.0f;
+      for (int i = 0; i < D; ++i) dot = fmaf(q[i], to_float<KV>(key[i]), dot);
+      const float score = lane < keys ? dot * qscale : -INFINITY;
+      const float m_new = fmaxf(m_run, group_max<kWave>(score));
+      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use), p = __builtin_amdgcn_exp2f(score - m_use);
+      m_run = m_new;
+      l = l * alpha + group_sum<kWave>(p);
+      o[0] *= alpha;
+      o[1] *= alpha;
+      for (int j = 0; j < keys; ++j) {
+        const float pj = read_lane(p, j);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          if (lane + c * kWave < D) o[c] = fmaf(pj, to_float<KV>(v[j * D + lane + c * kWave]), o[c]);
+      }
+    }
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int dim = lane + c * kWave;
+      const float x = o[c] * inv;
+      const int64_t off = row * a.out_stride + h * D + dim;
+      if (a.out && dim < D) a.out[off] = x;
+      if (a.out_split.hi) {
+        const float mx = group_max<kSplitChunkFine>(dim < D ? fabsf(x) : 0.0f);
+        int e = 0;
+        frexpf(mx, &e);  // e = 0 for a zero chunk
+        e = max(e, -100);
+        const float xs = x * ldexpf(1.0f, 15 - e);
+        const _Float16 hi = static_cast<_Float16>(xs), lo = static_cast<_Float16>(xs - static_cast<float>(hi));
+        if (dim < D) {
+          __builtin_memcpy(a.out_split.hi + off, &hi, 2);
+          __builtin_memcpy(a.out_split.lo + off, &lo, 2);
+          if (dim % kSplitChunkFine == 0)
+            a.out_split.inv[row * (a.hq * D / kSplitChunkFine) + (h * D + dim) / kSplitChunkFine] = ldexpf(1.0f, e - 15);
+        }
+      }
+    }
+  }
+}
+
 // Block = 32 queries x kHeads query heads of one KV group; its 8 waves are 2
 // heads x S = 4 key ranges, wave (s, hb) taking the 32-key tiles s, s + S, ...
 // of the block's causal range for head hb with its own online softmax.  The
@@ -212,6 +306,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   constexpr int DJ = D / 16, DT = D / 32;
   static_assert(2 * kTileChunks % kGroupThreads == 0 && kTileChunks % kWave == 0, "tile split over the group");
   __shared__ __align__(16) char lds[kLdsBytes];
+  __shared__ int bad[kWaves];
 
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -433,6 +528,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   }
   add_pv();
 
+  if (block_not_finite(ot, l_part, bad, wave, lane)) {
+    attend_rows_plainly<__half, D, HB, kPool>(a, s, lane, h, b, q0);
+    return;
+  }
   merge_and_write<D, HB>(a, ot, m_run, l_part, reinterpret_cast<float*>(lds), s, hb, lane, h, b, q0);
 }
 
@@ -451,8 +550,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // What bounds it: 36 products of 32 cycles a tile and head for d = 96 (1,152
 // cycles, where products of fp32 operands would take 6,144), and the splits' and
 // the softmax's vector instructions beside them.  prefill.hip's kernel / this
-// one, 8 query heads on 2: d 96, 2,000 rows 118.9 / 90.6 us, 4,096 rows 398.1 /
-// 173.2, 3,000 rows after 1,111 keys 349.8 / 174.6; d 64 77.6 / 71.5, 248.3 /
+// one, 8 query heads on 2: d 96, 2,000 rows 118.9 / 89.3 us, 4,096 rows 398.1 /
+// 170.5, 3,000 rows after 1,111 keys 349.8 / 171.3; d 64 77.6 / 71.5, 248.3 /
 // 136.5, 222.4 / 137.6.  Error against 64 bits of each dimension, of its own
 // largest value (d 96, 2,000 rows after 2,000 keys): 2.0e-6 / 1.1e-6; with V's
 // dimensions spread over 2^16 1.9e-6 / 1.1e-6, its keys over 2^20 2.2e-6 /
@@ -482,6 +581,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   constexpr int kMinScoreExp = -40;
   constexpr int kMinValueExp = -100;
   __shared__ __align__(16) char lds[kLdsBytes];
+  __shared__ int bad[kWaves];
   __shared__ __align__(16) int k_exp[2][S][HB], v_exp[2][S][HB];
 
   const int lane = threadIdx.x % kWave;
@@ -506,8 +606,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
     const int kcol = 32 * u + lane % 8 * 4, vcol = C * hb + (lane + u * kWave) % (C / 4) * 4;
-    koff[u] = krow * D + kcol;
-    kpos[u] = tile_chunk<D>(krow, kcol / 8) * 16 + kcol % 8 * 2;
+    // (Of d 96 the swizzle permutes groups of 4 chunks: each piece alike.)
+    koff[u] = u > 0 ? koff[0] + 32 * u : krow * D + kcol;
+    kpos[u] = D == 96 && u > 0 ? kpos[0] + 64 * u : tile_chunk<D>(krow, kcol / 8) * 16 + kcol % 8 * 2;
     voff[u] = vrow(u) * D + vcol;
     vpos[u] = tile_chunk<D>(vrow(u), vcol / 8) * 16 + vcol % 8 * 2;
   }
@@ -524,8 +625,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const int limit = last_key - t0;  // rows past the last key are masked, any key's row will do
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      uint32_t off = whole[u];
-      if (limit < kKeyTile - 1) off -= static_cast<uint32_t>(max(row(u) - limit, 0) * D);  // wave-uniform branch
+      int off = whole[u];
+      if (limit < kKeyTile - 1) off -= max(row(u) - limit, 0) * D;  // wave-uniform branch
       r[u] = *reinterpret_cast<const f32x4*>(base + off);
     }
   };
@@ -720,6 +821,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     for (int j = 0; j < DT; ++j) ot[j] *= alpha;
   }
   add_pv((n_iter - 1) & 1);
+  if (block_not_finite(ot, l_part, bad, wave, lane)) {
+    attend_rows_plainly<float, D, HB, kPool>(a, s, lane, h, b, q0);
+    return;
+  }
   merge_and_write<D, HB>(a, ot, m_run, l_part, reinterpret_cast<float*>(lds), s, hb, lane, h, b, q0);
 }
 

@@ -321,6 +321,47 @@ def test_prefill_attention_f32_keeps_small_dims(gpu, d, hq, hkv, start, T):
         assert err.max() < 5e-6, (h, int(err.argmax()), float(err.max()))
 
 
+@pytest.mark.parametrize("kv", ["f16", "f32"])
+@pytest.mark.parametrize("d", [64, 96])
+def test_prefill_attention_many_rows_confines_infinities(gpu, d, kv):
+    # An infinite value reaches its own dim of its own and later queries, a NaN
+    # value likewise; an infinite key makes a score of -inf, which counts for
+    # nothing, or of +inf, whose row is NaN.  All else is as without them.
+    mmr = gpu
+    hq, hkv, start, T = 8, 2, 40, 2000
+    print(f"[case] prefill attention infinities d={d} kv={kv}", flush=True)
+    rng = np.random.default_rng(d)
+    n = start + T
+    dt = np.float16 if kv == "f16" else np.float32
+    k = rng.standard_normal((hkv, n, d)).astype(dt)
+    v = (4 * rng.standard_normal((hkv, n, d))).astype(dt)
+    q = rng.standard_normal((T, hq, d)).astype(np.float32)
+    planted = v.copy()
+    planted[0, 1005, 7], planted[0, 1790, 40] = np.inf, np.nan
+    k[1, 1500, 9] = -np.inf
+    cache = mmr.KvCache(hkv, d, n, mmr.KV_F16 if kv == "f16" else mmr.KV_F32)
+    cache.upload(k, planted)
+    dq, out = mmr.DeviceArray.from_numpy(q.reshape(T, hq * d)), mmr.DeviceArray((T, hq * d), np.float32)
+    mmr.prefill_attention(dq, cache, start, T, hq, hkv, d, out)
+    got = out.numpy().reshape(T, hq, d)
+    position = start + np.arange(T)
+    hidden = np.arange(n)[None, :] > position[:, None]
+    with np.errstate(invalid="ignore"):
+        for h in range(hq):
+            g = h // (hq // hkv)
+            s = q[:, h].astype(np.float64) @ k[g].astype(np.float64).T / np.sqrt(d)
+            s[hidden] = -np.inf
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            ref = p @ v[g].astype(np.float64) / p.sum(axis=1, keepdims=True)
+            if g == 0:
+                ref[position >= 1005, 7] = np.inf
+                ref[position >= 1790, 40] = np.nan
+            np.testing.assert_array_equal(np.isnan(got[:, h]), np.isnan(ref))
+            np.testing.assert_array_equal(np.isposinf(got[:, h]), np.isposinf(ref))
+            finite = np.isfinite(ref)
+            assert 0 < finite.sum() and np.abs(got[:, h] - ref)[finite].max() < 1e-5 * np.abs(ref[finite]).max(), h
+
+
 def synth_model(mmr, g):
     return mmr.Model.synthetic(mmr.make_config(**g["config"]), g["seed"], g["std"], g["round_fp16"])
 
