@@ -207,6 +207,33 @@ def test_prefill_attention_group_sizes(gpu, oracle, hq, hkv):
         assert rel_err(got[t], ref) < TOL, t
 
 
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+def test_prefill_attention_few_rows_keep_q_exact(gpu, d):
+    # the 16-query kernel over an fp16 cache against 64 bits: q and p carry 22
+    # bits, sums are fp32 over at most 300 keys, so 1e-5 of the largest value; a
+    # q element whose two planes do not belong together is 1e-4
+    mmr = gpu
+    hq, hkv, T = 8, 2, 300
+    print(f"[case] prefill attention few rows d={d}", flush=True)
+    rng = np.random.default_rng(d)
+    k = rng.standard_normal((hkv, T, d)).astype(np.float16)
+    v = rng.standard_normal((hkv, T, d)).astype(np.float16)
+    q = (2 * rng.standard_normal((T, hq, d))).astype(np.float32)
+    cache = mmr.KvCache(hkv, d, T, mmr.KV_F16)
+    cache.upload(k, v)
+    dq, out = mmr.DeviceArray.from_numpy(q.reshape(T, hq * d)), mmr.DeviceArray((T, hq * d), np.float32)
+    mmr.prefill_attention(dq, cache, 0, T, hq, hkv, d, out)
+    got = out.numpy().reshape(T, hq, d)
+    hidden = np.triu(np.ones((T, T), bool), 1)
+    for h in range(hq):
+        g = h // (hq // hkv)
+        s = q[:, h].astype(np.float64) @ k[g].astype(np.float64).T / np.sqrt(d)
+        s[hidden] = -np.inf
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        ref = p @ v[g].astype(np.float64) / p.sum(axis=1, keepdims=True)
+        assert rel_err(got[:, h], ref) < 1e-5, h
+
+
 @pytest.mark.parametrize("d", [32, 64, 96])
 @pytest.mark.parametrize("hq,hkv,start,T", [(16, 2, 0, 449), (16, 2, 37, 480), (8, 2, 1000, 641), (8, 4, 511, 930),
                                             (12, 2, 20, 1300)])
