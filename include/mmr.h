@@ -102,6 +102,11 @@ int mmr_prefill_partial_floats(const mmr_config* config, int64_t chunk_rows, int
 /* Test aid, no reference counterpart (host arithmetic, no device needed):
  * whether an unsplit m x n x k product takes the 128 x 256 tiles for many rows. */
 int mmr_gemm_many_rows(int64_t m, int64_t n, int64_t k, int* many_rows);
+/* Test aid, no reference counterpart (host arithmetic, no device needed):
+ * whether causal attention of `tokens` rows from position `start` on, of each of
+ * `seqs` sequences, takes the 32-query kernels for many rows. */
+int mmr_prefill_attention_many_rows(int64_t q_heads, int64_t kv_heads, int64_t head_dim, int kv_dtype, int64_t start,
+                                    int64_t tokens, int64_t seqs, int* many_rows);
 /* Test aid, no reference counterpart: the (W row block, K chunk) that block
  * `block` of a batched split-K GEMM launch with grid (row_blocks, chunks)
  * computes (the blocks of one K chunk are placed on one XCD where chunks is a

@@ -292,6 +292,25 @@ int mmr_gemm_many_rows(int64_t m, int64_t n, int64_t k, int* many_rows) {
     *many_rows = mmr::gemm_rows_unsplit(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
   });
 }
+int mmr_prefill_attention_many_rows(int64_t q_heads, int64_t kv_heads, int64_t head_dim, int kv_dtype, int64_t start,
+                                    int64_t tokens, int64_t seqs, int* many_rows) {
+  return guarded([&] {
+    require(many_rows, "null result");
+    require(kv_dtype == MMR_KV_F16 || kv_dtype == MMR_KV_F32, "unknown kv dtype");
+    require(q_heads > 0 && kv_heads > 0 && head_dim > 0 && q_heads <= INT32_MAX && kv_heads <= INT32_MAX &&
+                head_dim <= INT32_MAX && start >= 0 && start <= INT32_MAX && tokens > 0 && tokens <= INT32_MAX &&
+                seqs > 0 && seqs <= INT32_MAX,
+            "shape out of range");
+    mmr::PrefillAttnArgs a;
+    a.hq = static_cast<int>(q_heads);
+    a.hkv = static_cast<int>(kv_heads);
+    a.d = static_cast<int>(head_dim);
+    a.start = static_cast<int>(start);
+    a.tokens = static_cast<int>(tokens);
+    a.seqs = static_cast<int>(seqs);
+    *many_rows = mmr::prefill_attention_many_rows(a, kv_dtype == MMR_KV_F16 ? mmr::kKvF16 : mmr::kKvF32);
+  });
+}
 int mmr_splitk_block_tile(int block, int row_blocks, int chunks, int* row_block, int* chunk) {
   return guarded([&] {
     require(row_block && chunk, "null argument");

@@ -838,36 +838,65 @@ static bool many_rows_shape(const PrefillAttnArgs& a, int heads) {
     return false;
   return a.hkv > 0 && a.hq % a.hkv == 0 && a.hq / a.hkv % heads == 0;
 }
-static int64_t many_rows_blocks(const PrefillAttnArgs& a, int heads) {
-  return int64_t{(a.tokens + kQueryTile - 1) / kQueryTile} * (a.hq / heads) * a.seqs;
-}
 
-// Enough rows for these kernels, against prefill.hip's, whose blocks are 16
-// queries x 1 head, one per CU.
-//
-// fp16 cache: that one's time steps up when its blocks pass 256, the CUs (512
-// rows for 8 heads); this one has a quarter as many blocks, with a longer start
-// and end, and wins once they fill about half the CUs, or sooner after a long
-// cached context, where the key loop is most of the time.  d 96 (16-query
-// kernel / this one): 512 rows 8.9 / 13.3 us, 700 rows 15.2 / 15.7, 1,000 rows
-// 22.2 / 18.0; after 2,000 cached keys 300 rows 21.9 / 28.3, 700 rows 43.7 /
-// 32.5.  d 64: 700 rows 11.4 / 12.5, 1,000 rows 15.1 / 14.6; after 2,000 keys
-// 700 rows 30.2 / 26.3.  (d 128 does not fit the registers of two waves per
-// SIMD.)
-//
-// fp32 cache: an eighth as many blocks.  8 heads, d 96: 1,000 rows (64 blocks)
-// 43.8 / 49.8, 2,000 rows (126) 118.9 / 88.5; after 2,000 keys 1,000 rows 114.2
-// / 126.3.  d 64: 1,000 rows 29.3 / 40.3, 2,000 rows 78.6 / 70.6; after 2,000
-// keys 1,000 rows 74.6 / 100.9.  (d 32, with a third of d 96's products to the
-// same softmax and splits, measured slower at all but 4,096 rows.)
-bool prefill_attention_many_rows(const PrefillAttnArgs& a, KvDtype kv) {
-  if (kv == kKvF16) {
-    if ((a.d != 32 && a.d != 64 && a.d != 96) || !many_rows_shape(a, kHeads)) return false;
-    const int64_t blocks = many_rows_blocks(a, kHeads);
-    return blocks >= 112 || (blocks >= 80 && a.start >= a.tokens);
+// The time of a launch as its blocks' rounds (one block per CU) times a block's
+// start and end and its keys.
+struct AttnCost {
+  float base, round, key;  // us
+  float us(int64_t blocks, float keys) const {
+    constexpr int64_t kCus = 256;
+    return base + static_cast<float>((blocks + kCus - 1) / kCus) * (round + key * keys);
   }
-  return kv == kKvF32 && (a.d == 64 || a.d == 96) && many_rows_shape(a, kHeads32) &&
-         many_rows_blocks(a, kHeads32) >= 120;
+};
+
+// These kernels against prefill.hip's, whose blocks are 16 queries x 1 head: an
+// eighth (fp32 cache) or a quarter as many blocks here, with a longer start and
+// end.  Either time steps up when the blocks pass a multiple of the 256 CUs,
+// for one sequence as for a batch of short ones.  The costs are fitted to kernel
+// times of 93 launches per row of the table, 8 query heads on 2, one sequence of
+// 64-4,096 rows after 0-6,000 keys and batches of 2-128 sequences of 8-1,500
+// rows; the choice by them takes 0.1% (d 32: 0.4, fp32 d 64: 0.3) more than the better
+// kernel of each, where a count of this kernel's blocks took 1.6-5.2%.  Some of
+// them (prefill.hip / this one), fp16 d 96: 64 sequences of 16 rows 10.2 / 11.1
+// us, of 24 19.6 / 12.1; 16 of 64 10.6 / 12.3, of 100 20.1 / 13.4; one of 512 rows
+// 8.9 / 13.3, of 700 after 2,000 keys 43.7 / 32.5; d 64: 64 of 33 14.5 / 18.4, 16 of
+// 160 14.8 / 18.2, of 255 24.8 / 21.4.  fp32 d 96: 64 of 16 11.7 / 13.4, of 24 21.5 /
+// 14.6; 8 of 200 28.3 / 21.6; one of 1,000 43.8 / 49.8, of 2,000 118.9 / 89.3; d 64:
+// 32 of 48 9.8 / 11.7, 16 of 255 38.8 / 22.1.  (fp16 d 128 does not fit the
+// registers of two waves per SIMD; d 32 on an fp32 cache, with a third of d 96's
+// products to the same softmax and splits, measured slower at all but 4,096 rows.)
+bool prefill_attention_many_rows(const PrefillAttnArgs& a, KvDtype kv) {
+  const bool f16 = kv == kKvF16;
+  const int heads = f16 ? kHeads : kHeads32;
+  if (!(f16 || kv == kKvF32) || !many_rows_shape(a, heads)) return false;
+  AttnCost few, many;
+  switch (a.d) {
+    case 32:
+      if (!f16) return false;
+      few = {3.0f, 0.9f, 0.0046f}, many = {5.0f, 2.0f, 0.0055f};
+      break;
+    case 64:
+      if (f16) {
+        few = {3.4f, 1.85f, 0.0055f}, many = {0.0f, 9.5f, 0.0068f};
+      } else {
+        few = {3.9f, 1.95f, 0.0152f}, many = {0.0f, 11.6f, 0.0370f};
+      }
+      break;
+    case 96:
+      if (f16) {
+        few = {2.2f, 4.2f, 0.0076f}, many = {0.0f, 11.8f, 0.0082f};
+      } else {
+        few = {2.9f, 4.7f, 0.0220f}, many = {0.0f, 15.6f, 0.0450f};
+      }
+      break;
+    default: return false;
+  }
+  const int64_t row_heads = static_cast<int64_t>(a.hq) * a.seqs;
+  const float start = static_cast<float>(a.start), tokens = static_cast<float>(a.tokens);
+  const int64_t few_blocks = (a.tokens + int64_t{15}) / 16 * row_heads;
+  const int64_t many_blocks = (a.tokens + int64_t{kQueryTile} - 1) / kQueryTile * (row_heads / heads);
+  // Keys of a block: the mean where there are many rounds, nearer the longest in one.
+  return many.us(many_blocks, start + 0.75f * tokens) < few.us(few_blocks, start + 0.5f * tokens);
 }
 
 namespace {

@@ -103,6 +103,7 @@ _SIGS = {
     "mmr_event_elapsed_ms": ([VP, VP, P_F32], C.c_int),
     "mmr_gemm_k_splits": ([I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
     "mmr_gemm_many_rows": ([I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
+    "mmr_prefill_attention_many_rows": ([I64, I64, I64, C.c_int, I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
     "mmr_prefill_partial_floats": ([C.POINTER(Config), I64, C.POINTER(I64)], C.c_int),
     "mmr_splitk_block_tile": ([C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)], C.c_int),
     "mmr_decode_attention_splits": ([I64, I64, C.POINTER(C.c_int)], C.c_int),
@@ -380,6 +381,15 @@ def gemm_many_rows(m: int, n: int, k: int) -> bool:
     """Whether an unsplit m x n x k product takes the 128 x 256 tiles for many rows (host arithmetic)."""
     out = C.c_int()
     check(_lib.mmr_gemm_many_rows(m, n, k, C.byref(out)))
+    return bool(out.value)
+
+
+def prefill_attention_many_rows(q_heads: int, kv_heads: int, head_dim: int, kv_dtype: int, start: int, tokens: int,
+                                seqs: int = 1) -> bool:
+    """Whether causal attention of these rows takes the 32-query kernels for many rows (host arithmetic)."""
+    out = C.c_int()
+    check(_lib.mmr_prefill_attention_many_rows(q_heads, kv_heads, head_dim, kv_dtype, start, tokens, seqs,
+                                               C.byref(out)))
     return bool(out.value)
 
 

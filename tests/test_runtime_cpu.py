@@ -221,6 +221,24 @@ def test_many_rows_tiles_need_rows_as_well_as_tiles(mmr, m, n, k, chosen):
     assert mmr.gemm_many_rows(m, n, k) is chosen
 
 
+@pytest.mark.parametrize("kv,d,start,tokens,seqs,many", [
+    ("f16", 96, 0, 512, 1, False), ("f16", 96, 0, 1000, 1, True), ("f16", 96, 2000, 300, 1, False),
+    ("f16", 96, 2000, 700, 1, True), ("f16", 96, 0, 16, 64, False), ("f16", 96, 0, 24, 64, True),
+    ("f16", 96, 0, 64, 16, False), ("f16", 96, 0, 100, 16, True), ("f16", 96, 0, 31, 32, False),
+    ("f16", 64, 0, 33, 64, False), ("f16", 64, 0, 160, 16, False), ("f16", 64, 0, 255, 16, True),
+    ("f16", 64, 0, 500, 8, True), ("f16", 32, 0, 127, 32, True), ("f16", 32, 0, 16, 64, False),
+    ("f32", 96, 0, 1000, 1, False), ("f32", 96, 0, 2000, 1, True), ("f32", 96, 0, 16, 64, False),
+    ("f32", 96, 0, 24, 64, True), ("f32", 96, 0, 200, 8, True), ("f32", 96, 0, 128, 8, False),
+    ("f32", 64, 0, 48, 32, False), ("f32", 64, 0, 255, 16, True), ("f32", 64, 0, 1000, 1, False),
+    ("f16", 128, 0, 4096, 1, False), ("f32", 128, 0, 4096, 1, False), ("f32", 32, 0, 4096, 1, False)])
+def test_prefill_attention_kernel_follows_rounds(mmr, kv, d, start, tokens, seqs, many):
+    # 8 query heads on 2, each as it measured: short sequences of a batch leave
+    # most of a 32-query tile empty, or take more rounds of blocks than they save.
+    kvd = mmr.KV_F16 if kv == "f16" else mmr.KV_F32
+    assert mmr.prefill_attention_many_rows(8, 2, d, kvd, start, tokens, seqs) is many
+    assert not mmr.prefill_attention_many_rows(3, 3, d, kvd, start, tokens, seqs)  # no heads to share K and V
+
+
 @pytest.mark.parametrize("head_dim,tile", [(96, 64), (64, 64), (128, 32)])
 def test_decode_split_buckets(mmr, head_dim, tile):
     # The decode step replays one graph per attention split count, and the KV
