@@ -102,6 +102,9 @@ int mmr_prefill_partial_floats(const mmr_config* config, int64_t chunk_rows, int
 /* Test aid, no reference counterpart (host arithmetic, no device needed):
  * whether an unsplit m x n x k product takes the 128 x 256 tiles for many rows. */
 int mmr_gemm_many_rows(int64_t m, int64_t n, int64_t k, int* many_rows);
+/* Test aid, no reference counterpart (host arithmetic, no device needed): the
+ * rows of a prefill pass when n rows run in equal passes of at most `most`. */
+int mmr_prefill_pass_rows(int64_t n, int64_t most, int64_t* rows);
 /* Test aid, no reference counterpart (host arithmetic, no device needed):
  * whether causal attention of `tokens` rows from position `start` on, of each of
  * `seqs` sequences, takes the 32-query kernels for many rows. */

@@ -292,6 +292,13 @@ int mmr_gemm_many_rows(int64_t m, int64_t n, int64_t k, int* many_rows) {
     *many_rows = mmr::gemm_rows_unsplit(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
   });
 }
+int mmr_prefill_pass_rows(int64_t n, int64_t most, int64_t* rows) {
+  return guarded([&] {
+    require(rows, "null result");
+    require(n > 0 && most > 0, "row count out of range");
+    *rows = prefill_pass_rows(n, most);
+  });
+}
 int mmr_prefill_attention_many_rows(int64_t q_heads, int64_t kv_heads, int64_t head_dim, int kv_dtype, int64_t start,
                                     int64_t tokens, int64_t seqs, int* many_rows) {
   return guarded([&] {

@@ -46,6 +46,9 @@ namespace minimind::model {
 constexpr int kBatchWarmBlocks = 0;
 constexpr int64_t kBatchWarmMaxBytes = int64_t{16} << 20;  // half the 32 MB of L2
 
+// Most prompt rows (over all sequences) of one pass of the prefill layers.
+constexpr int64_t kPromptRows = 4096;
+
 struct BatchDeviceState {
   std::shared_ptr<const DeviceModel> model;
   mmr::KvDtype kv = mmr::kKvF16;
@@ -78,6 +81,8 @@ struct BatchDeviceState {
   std::map<int, hipGraphExec_t> graphs;
   bool use_graphs = true;
   bool prompt_tokenwise = false;  // prompts through the decode steps (comparison switch)
+  int64_t prompt_rows = kPromptRows;
+  bool register_staged = false;   // prompt GEMMs on the register-staged kernel only (comparison switch)
   // L2-warming blocks of the residual + norm launches (0 = none): the one
   // after the O projection loads gate_up and down, the one after down the
   // next layer's qkv (after the last layer the lm_head's).
@@ -333,24 +338,24 @@ void enqueue_batch_step_kernels(const BatchDeviceState& s, int splits) {
             "batch logits + argmax");
 }
 
-// Prompt rows (over all sequences) that one pass of the prefill layers takes.
-constexpr int64_t kPromptRows = 4096;
 // Fewest prompt tokens worth the prefill layers: one pass of them takes about
 // as long as this many steps.
 constexpr int64_t kMinPromptRows = 4;
 
 // Tokens 0 .. count - 1 of every sequence into the KV pools through the
-// batched prefill layers: rows [sequence][token], kPromptRows rows at a time.
+// batched prefill layers: rows [sequence][token], in equal passes of at most
+// prompt_rows rows.
 // Nothing is predicted: the last layer stops after its keys and values.
 void enqueue_prompt_rows(BatchDeviceState& s, int64_t count) {
   const DeviceModel& m = *s.model;
   const auto& c = m.cfg;
-  const int64_t chunk = std::min(count, std::max<int64_t>(1, kPromptRows / s.batch));
+  const int64_t chunk = prefill_pass_rows(count, std::max<int64_t>(1, s.prompt_rows / s.batch));
   const std::size_t h_bytes = Arena::round_up(static_cast<std::size_t>(s.batch * chunk * c.hidden_size) * sizeof(float));
   s.prompt_buf.reset(h_bytes + prefill_scratch_bytes(c, s.batch * chunk));
   float* h = static_cast<float*>(s.prompt_buf.data());
-  const PrefillScratch scratch =
+  PrefillScratch scratch =
       carve_prefill_scratch(c, s.batch * chunk, static_cast<char*>(s.prompt_buf.data()) + h_bytes);
+  scratch.register_staged = s.register_staged;
   for (int64_t first = 0; first < count; first += chunk) {
     const int tokens = static_cast<int>(std::min(chunk, count - first));
     const int rows = static_cast<int>(s.batch) * tokens;
@@ -432,6 +437,9 @@ BatchState LanguageModel::make_batch_state(int64_t batch, int64_t capacity, KvCa
   s->use_graphs = !(nog && nog[0] == '1');
   const char* pt = std::getenv("MMR_PREFILL_TOKENWISE");
   s->prompt_tokenwise = pt && pt[0] == '1';
+  if (const char* pc = std::getenv("MMR_PREFILL_CHUNK")) s->prompt_rows = std::max<int64_t>(1, std::atoll(pc));
+  const char* rs = std::getenv("MMR_GEMM_REGISTER_STAGED");
+  s->register_staged = rs && rs[0] == '1';
   const int64_t H = c.hidden_size, D = c.head_dim, Hq = c.num_attention_heads, Hkv = c.num_key_value_heads;
   const int64_t F = c.intermediate_size, V = c.vocab_size;
   const int64_t pages = batch * s->pages_per_seq;

@@ -852,8 +852,7 @@ void LanguageModel::enqueue_prefill(DecoderState& state, const std::vector<int32
   float* h = s.pf_h;
   const PrefillScratch* scratch = &s.pf;
   if (n > chunk && s.pf_long > chunk) {
-    const int64_t passes = (n + s.pf_long - 1) / s.pf_long;
-    chunk = (n + passes - 1) / passes;
+    chunk = prefill_pass_rows(n, s.pf_long);
     if (s.pf_long_scratch.rows < chunk) reserve_long_prefill(s, chunk);
     h = s.pf_long_h;
     scratch = &s.pf_long_scratch;

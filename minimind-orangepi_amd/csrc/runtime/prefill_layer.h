@@ -41,6 +41,13 @@ struct PrefillScratch {
 std::size_t prefill_scratch_bytes(const MiniMindConfig& c, int64_t rows);
 PrefillScratch carve_prefill_scratch(const MiniMindConfig& c, int64_t rows, void* base);
 
+// Rows of a pass when n rows run in as few equal passes of at most `most` as they
+// need (the last pass may be shorter by less than the number of passes).
+inline int64_t prefill_pass_rows(int64_t n, int64_t most) {
+  const int64_t passes = (n + most - 1) / most;
+  return (n + passes - 1) / passes;
+}
+
 // Layer input norm of the first layer: h [rows][H] normalised with `norm`
 // into the scratch (the form the QKV GEMM reads for this row count).
 void enqueue_prefill_input_norm(const MiniMindConfig& c, const PrefillScratch& s, int rows, const float* h,

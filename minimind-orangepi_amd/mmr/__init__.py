@@ -103,6 +103,7 @@ _SIGS = {
     "mmr_event_elapsed_ms": ([VP, VP, P_F32], C.c_int),
     "mmr_gemm_k_splits": ([I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
     "mmr_gemm_many_rows": ([I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
+    "mmr_prefill_pass_rows": ([I64, I64, C.POINTER(I64)], C.c_int),
     "mmr_prefill_attention_many_rows": ([I64, I64, I64, C.c_int, I64, I64, I64, C.POINTER(C.c_int)], C.c_int),
     "mmr_prefill_partial_floats": ([C.POINTER(Config), I64, C.POINTER(I64)], C.c_int),
     "mmr_splitk_block_tile": ([C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)], C.c_int),
@@ -391,6 +392,13 @@ def prefill_attention_many_rows(q_heads: int, kv_heads: int, head_dim: int, kv_d
     check(_lib.mmr_prefill_attention_many_rows(q_heads, kv_heads, head_dim, kv_dtype, start, tokens, seqs,
                                                C.byref(out)))
     return bool(out.value)
+
+
+def prefill_pass_rows(n: int, most: int) -> int:
+    """Rows of a prefill pass when n rows run in equal passes of at most `most` (host arithmetic)."""
+    out = I64()
+    check(_lib.mmr_prefill_pass_rows(n, most, C.byref(out)))
+    return out.value
 
 
 def splitk_block_tile(block: int, row_blocks: int, chunks: int) -> tuple[int, int]:

@@ -132,9 +132,8 @@ def test_batch_sizes_across_gemm_paths(gpu, batch):
 def test_batch_prompt_rows_match_tokenwise(gpu, monkeypatch, batch, low, high, kv):
     # the prompts through the prefill layers against the same prompts through
     # the steps (MMR_PREFILL_TOKENWISE): the fewest rows that take them (4);
-    # 699 rows of two sequences (the many-rows attention over pages); 33 and
-    # 300 sequences, whose rows run in two and three passes (4,096 rows over
-    # the batch a pass), the last of them ragged
+    # 699 rows of two sequences; 33 and 300 sequences, whose rows run in two and
+    # three passes (4,096 rows over the batch a pass), the last of them ragged
     mmr = gpu
     print(f"[case] batch prompt rows B={batch} {low}..{high} kv={kv}", flush=True)
     g = load_golden("mini")
@@ -157,6 +156,28 @@ def test_batch_prompt_rows_match_tokenwise(gpu, monkeypatch, batch, low, high, k
     for b in sorted({0, 1, batch // 2, batch - 1}):
         np.testing.assert_array_equal(rows.read_sequence(b, 0, last + 1), tok.read_sequence(b, 0, last + 1))
         assert rel_err(rows.read_logits(b), tok.read_logits(b)) < 1e-4, b
+
+
+@pytest.mark.parametrize("switch,value", [("MMR_GEMM_REGISTER_STAGED", "1"), ("MMR_PREFILL_CHUNK", "100")])
+def test_batch_prompt_rows_follow_the_switches(gpu, monkeypatch, switch, value):
+    # 5 sequences of 61 shared tokens: the other GEMM kernel, and passes of 16
+    # tokens of each (80 rows), the last of 13, give the same answer
+    mmr = gpu
+    print(f"[case] batch prompt rows {switch}={value}", flush=True)
+    g = load_golden("mini")
+    m = synth_model(mmr, g)
+    rng = np.random.default_rng(9)
+    prompts = [[int(t) for t in rng.integers(0, g["config"]["vocab_size"], 62 + b)] for b in range(5)]
+    plain = m.make_batch_state(5, 80, mmr.KV_F32)
+    monkeypatch.setenv(switch, value)
+    other = m.make_batch_state(5, 80, mmr.KV_F32)
+    for st in (plain, other):
+        st.prefill(prompts)
+        st.decode(4)
+        st.synchronize()
+    for b in range(5):
+        np.testing.assert_array_equal(other.read_sequence(b, 0, 71), plain.read_sequence(b, 0, 71))
+        assert rel_err(other.read_logits(b), plain.read_logits(b)) < 1e-5, b
 
 
 def test_batch_reproduces_reference_golden(gpu):

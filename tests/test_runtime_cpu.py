@@ -221,6 +221,18 @@ def test_many_rows_tiles_need_rows_as_well_as_tiles(mmr, m, n, k, chosen):
     assert mmr.gemm_many_rows(m, n, k) is chosen
 
 
+def test_prefill_passes_are_equal(mmr):
+    # As few passes as fit and none of them a remainder: 125 tokens of 33
+    # sequences, 124 of which fit a pass of 4,096 rows, run as 63 + 62.
+    assert mmr.prefill_pass_rows(125, 4096 // 33) == 63
+    for n in (1, 2, 511, 512, 513, 4096, 4097, 6000, 8193):
+        for most in (1, 7, 64, 512, 4096):
+            rows = mmr.prefill_pass_rows(n, most)
+            passes = -(-n // most)
+            assert 1 <= rows <= most and -(-n // rows) <= passes
+            assert n - (passes - 1) * rows > rows - passes  # the last pass
+
+
 @pytest.mark.parametrize("kv,d,start,tokens,seqs,many", [
     ("f16", 96, 0, 512, 1, False), ("f16", 96, 0, 1000, 1, True), ("f16", 96, 2000, 300, 1, False),
     ("f16", 96, 2000, 700, 1, True), ("f16", 96, 0, 16, 64, False), ("f16", 96, 0, 24, 64, True),
