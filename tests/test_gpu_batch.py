@@ -158,6 +158,41 @@ def test_batch_prompt_rows_match_tokenwise(gpu, monkeypatch, batch, low, high, k
         assert rel_err(rows.read_logits(b), tok.read_logits(b)) < 1e-4, b
 
 
+@pytest.mark.parametrize("d,kv,batch,low,high", [(64, "f32", 64, 101, 110), (96, "f32", 64, 101, 110),
+                                                 (64, "f16", 16, 501, 510), (96, "f16", 64, 101, 110)])
+def test_batch_prompt_rows_take_many_rows_attention(gpu, monkeypatch, d, kv, batch, low, high):
+    # 8 query heads on 2: the 32-query attention kernels over a batch's pages, in
+    # two passes of the prompts (the second after cached rows), a last query
+    # tile that is not full; against the prompts through the steps
+    mmr = gpu
+    print(f"[case] batch many-rows attention B={batch} {low}..{high} d={d} kv={kv}", flush=True)
+    kvd = mmr.KV_F16 if kv == "f16" else mmr.KV_F32
+    cfg = mmr.make_config(hidden_size=8 * d, num_hidden_layers=3, num_attention_heads=8, num_key_value_heads=2,
+                          head_dim=d, intermediate_size=512, vocab_size=512, max_position_embeddings=1024,
+                          rms_norm_eps=1e-5, rope_theta=1e6, tie_word_embeddings=1)
+    m = mmr.Model.synthetic(cfg, 5, 0.02, True)
+    passes = -(-(low - 1) * batch // 4096)
+    first = mmr.prefill_pass_rows(low - 1, 4096 // batch)
+    assert passes == 2 and first % 32 != 0
+    for start, tokens in ((0, first), (first, low - 1 - first)):
+        assert mmr.prefill_attention_many_rows(8, 2, d, kvd, start, tokens, batch)
+    rng = np.random.default_rng(batch + low)
+    lengths = [low] + [int(n) for n in rng.integers(low, high + 1, batch - 1)]
+    prompts = [[int(t) for t in rng.integers(0, 512, n)] for n in lengths]
+    last = max(lengths) + 4
+    monkeypatch.setenv("MMR_PREFILL_TOKENWISE", "1")
+    tok = m.make_batch_state(batch, last, kvd)
+    monkeypatch.delenv("MMR_PREFILL_TOKENWISE")
+    rows = m.make_batch_state(batch, last, kvd)
+    for st in (tok, rows):
+        st.prefill(prompts)
+        st.decode(4)
+        st.synchronize()
+    for b in sorted({0, 1, batch // 2, batch - 1}):
+        np.testing.assert_array_equal(rows.read_sequence(b, 0, last + 1), tok.read_sequence(b, 0, last + 1))
+        assert rel_err(rows.read_logits(b), tok.read_logits(b)) < (1e-4 if kv == "f32" else 1e-3), b
+
+
 @pytest.mark.parametrize("switch,value", [("MMR_GEMM_REGISTER_STAGED", "1"), ("MMR_PREFILL_CHUNK", "100")])
 def test_batch_prompt_rows_follow_the_switches(gpu, monkeypatch, switch, value):
     # 5 sequences of 61 shared tokens: the other GEMM kernel, and passes of 16
