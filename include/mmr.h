@@ -399,7 +399,8 @@ int mmr_state_position(const mmr_state* state, int64_t* position);
  * NULL. */
 int mmr_state_kv_backed(const mmr_state* state, int64_t* tokens, uint64_t* device_bytes);
 /* Back KV positions [0, positions) now (at most the capacity), so decoding up
- * to there allocates nothing (allocates; synchronous). */
+ * to there allocates nothing (allocates; synchronous).  A prompt of over 512
+ * tokens may still allocate, see mmr_enqueue_prefill. */
 int mmr_state_reserve(const mmr_model* model, mmr_state* state, int64_t positions);
 int mmr_state_stream(const mmr_state* state, mmr_stream_t* stream);
 int mmr_state_reset(const mmr_model* model, mmr_state* state);
@@ -412,7 +413,11 @@ int mmr_prefill_next_token(const mmr_model* model, mmr_state* state, const int32
 int mmr_generate(const mmr_model* model, const int32_t* prompt, int64_t n, int64_t max_new_tokens, int32_t* out,
                  int64_t* out_count);
 
-/* Device-resident loop (no host round trip per token). */
+/* Device-resident loop (no host round trip per token).  The first prompt of over
+ * 512 tokens (in one call) allocates buffers for passes of up to 4,096 tokens,
+ * about 49 KB a token of a pass for MiniMind2 (199 MB at most), which the state
+ * keeps and a longer prompt may replace; if the device does not have the memory,
+ * the prompt runs in passes of 512 on the buffers that the state has. */
 int mmr_enqueue_prefill(const mmr_model* model, mmr_state* state, const int32_t* prompt, int64_t n);
 int mmr_enqueue_decode(const mmr_model* model, mmr_state* state, int64_t steps, int32_t first_token);
 int mmr_state_synchronize(const mmr_model* model, mmr_state* state);

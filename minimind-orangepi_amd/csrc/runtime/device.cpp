@@ -14,6 +14,20 @@ void DeviceBuffer::reset(std::size_t bytes) {
   bytes_ = bytes;
 }
 
+bool DeviceBuffer::try_reset(std::size_t bytes) {
+  release();
+  if (bytes == 0) return true;
+  const hipError_t status = hipMalloc(&data_, bytes);
+  if (status == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    data_ = nullptr;
+    return false;
+  }
+  check_hip(status, "hipMalloc");
+  bytes_ = bytes;
+  return true;
+}
+
 void DeviceBuffer::release() noexcept {
   if (data_) (void)hipFree(data_);
   data_ = nullptr;

@@ -44,6 +44,9 @@ class DeviceBuffer {
   void* data() const noexcept { return data_; }
   std::size_t bytes() const noexcept { return bytes_; }
   void reset(std::size_t bytes);
+  // The same where the caller has another way: false (and no buffer) if the
+  // device does not have the memory.
+  bool try_reset(std::size_t bytes);
 
  private:
   void release() noexcept;

@@ -81,8 +81,9 @@ struct DeviceState {
   float* pf_h = nullptr;    // [chunk][H] residual stream
   PrefillScratch pf;        // the layer's scratch for pf_chunk rows
   // The same for longer prompts (up to pf_long rows a pass), allocated by the
-  // first prompt that needs it.
+  // first prompt that needs it where the memory is there.
   int64_t pf_long = 0;
+  std::size_t pf_long_limit = SIZE_MAX;  // bytes
   DeviceBuffer pf_long_buf;
   float* pf_long_h = nullptr;
   PrefillScratch pf_long_scratch;
@@ -124,9 +125,11 @@ constexpr int kMaxSplits = 512;
 // in as few equal passes of up to kPrefillLongChunk rows as they need, whose
 // larger GEMMs and attention launches fill the GPU (6,000 tokens of MiniMind2,
 // fp16 cache: passes of 512 rows 15.3 ms, 2,048 8.4 ms, 6,000 7.1 ms, before
-// the many-rows GEMM), on buffers of about 40 KB a row.
+// the many-rows GEMM), on buffers of their own: about 49 KB a row of MiniMind2
+// (199 MB for 4,096), grown in steps of kPrefillLongStep rows.
 constexpr int64_t kPrefillChunk = 512;
 constexpr int64_t kPrefillLongChunk = 4096;
+constexpr int64_t kPrefillLongStep = 512;
 
 void require_size(const std::vector<float>& v, int64_t expected, const std::string& name) {
   if (static_cast<int64_t>(v.size()) != expected) throw std::invalid_argument(name + " has invalid size");
@@ -342,6 +345,7 @@ DecoderState LanguageModel::make_state(int64_t capacity, KvCacheDtype kv) const 
   ar.plan(device_->plan_lm.blocks * 4);
   int64_t chunk = kPrefillChunk;
   s->pf_long = kPrefillLongChunk;
+  s->pf_long_limit = prefill_buffer_limit();
   if (const char* pc = std::getenv("MMR_PREFILL_CHUNK")) s->pf_long = chunk = std::max<int64_t>(1, std::atoll(pc));
   s->pf_chunk = s->prefill_tokenwise ? 0 : std::min<int64_t>(capacity, chunk);
   const int64_t C = s->pf_chunk;
@@ -710,15 +714,20 @@ void enqueue_prefill_chunk(const DeviceState& s, int64_t start, int64_t n, float
 }
 
 // Buffers of a prefill pass of `rows` rows (the stream is idle: nothing reads
-// the previous ones).
-void reserve_long_prefill(DeviceState& s, int64_t rows) {
+// the previous ones); false if the memory is not to be had.
+bool reserve_long_prefill(DeviceState& s, int64_t rows) {
+  if (s.pf_long_scratch.rows >= rows) return true;
   const auto& c = s.model->cfg;
+  rows = std::min((rows + kPrefillLongStep - 1) / kPrefillLongStep * kPrefillLongStep, s.pf_long);
   const std::size_t h_bytes = Arena::round_up(static_cast<std::size_t>(rows * c.hidden_size) * sizeof(float));
+  const std::size_t bytes = h_bytes + prefill_scratch_bytes(c, rows);
+  if (bytes > s.pf_long_limit) return false;
   s.pf_long_scratch = PrefillScratch{};
-  s.pf_long_buf.reset(h_bytes + prefill_scratch_bytes(c, rows));
+  if (!s.pf_long_buf.try_reset(bytes)) return false;
   s.pf_long_h = static_cast<float*>(s.pf_long_buf.data());
   s.pf_long_scratch = carve_prefill_scratch(c, rows, static_cast<char*>(s.pf_long_buf.data()) + h_bytes);
   s.pf_long_scratch.register_staged = s.pf.register_staged;
+  return true;
 }
 
 // `steps` consecutive decode steps with one attention split count, as one
@@ -851,9 +860,9 @@ void LanguageModel::enqueue_prefill(DecoderState& state, const std::vector<int32
   int64_t last_rows = 0, chunk = s.pf_chunk;
   float* h = s.pf_h;
   const PrefillScratch* scratch = &s.pf;
-  if (n > chunk && s.pf_long > chunk) {
-    chunk = prefill_pass_rows(n, s.pf_long);
-    if (s.pf_long_scratch.rows < chunk) reserve_long_prefill(s, chunk);
+  const int64_t long_chunk = prefill_pass_rows(n, std::max(s.pf_long, chunk));
+  if (n > chunk && s.pf_long > chunk && reserve_long_prefill(s, long_chunk)) {
+    chunk = long_chunk;
     h = s.pf_long_h;
     scratch = &s.pf_long_scratch;
   }

@@ -3,6 +3,8 @@
 #include "device.h"
 
 #include <algorithm>
+#include <cstdint>
+#include <cstdlib>
 #include <stdexcept>
 
 namespace minimind::model {
@@ -77,6 +79,11 @@ std::size_t prefill_scratch_bytes(const MiniMindConfig& c, int64_t rows) {
   Carver cv;
   (void)carve(c, rows, cv);
   return cv.used;
+}
+
+std::size_t prefill_buffer_limit() {
+  const char* mb = std::getenv("MMR_PREFILL_BUFFER_MB");
+  return mb ? static_cast<std::size_t>(std::max<long long>(0, std::atoll(mb))) << 20 : SIZE_MAX;
 }
 
 PrefillScratch carve_prefill_scratch(const MiniMindConfig& c, int64_t rows, void* base) {

@@ -48,6 +48,10 @@ inline int64_t prefill_pass_rows(int64_t n, int64_t most) {
   return (n + passes - 1) / passes;
 }
 
+// Most bytes that the pass buffers of one long prompt, or of one batch's
+// prompts, may take (MMR_PREFILL_BUFFER_MB; no limit by default).
+std::size_t prefill_buffer_limit();
+
 // Layer input norm of the first layer: h [rows][H] normalised with `norm`
 // into the scratch (the form the QKV GEMM reads for this row count).
 void enqueue_prefill_input_norm(const MiniMindConfig& c, const PrefillScratch& s, int rows, const float* h,

@@ -524,6 +524,33 @@ def test_minimind2_long_passes_match_chunks(gpu, monkeypatch, prompt_len):
     assert passes.read_sequence(prompt_len, 1).tolist() == chunks.read_sequence(prompt_len, 1).tolist()
 
 
+def test_long_prompts_without_the_pass_buffers(gpu, monkeypatch):
+    # no memory for the buffers of long passes (and, in a second state, for those
+    # of the longer of two prompts): passes of 512 tokens on the state's own,
+    # with the bits of such passes
+    mmr = gpu
+    print("[case] long prompts without the pass buffers", flush=True)
+    g = load_golden("mini")
+    m = synth_model(mmr, g)
+    rng = np.random.default_rng(4)
+    first, second = ([int(t) for t in rng.integers(0, g["config"]["vocab_size"], n)] for n in (700, 1300))
+    logits = {}
+    for name, switch, value in (("chunks", "MMR_PREFILL_CHUNK", "512"), ("none", "MMR_PREFILL_BUFFER_MB", "0"),
+                                ("some", "MMR_PREFILL_BUFFER_MB", "16")):
+        monkeypatch.setenv(switch, value)
+        st = m.make_state(2048, mmr.KV_F32)
+        monkeypatch.delenv(switch)
+        st.enqueue_prefill(first)
+        one = st.read_logits()
+        st.enqueue_prefill(second)
+        st.enqueue_decode(3)
+        logits[name] = one, st.read_logits()
+    for one, two in zip(logits["chunks"], logits["none"]):
+        np.testing.assert_array_equal(two, one)
+    for one, two in zip(logits["chunks"], logits["some"]):
+        assert rel_err(two, one) < 1e-4
+
+
 def test_gemm_kernels_agree(gpu, monkeypatch):
     # the direct-to-LDS GEMM (pre-split A, K % 64 == 0) against the
     # register-staged one (MMR_GEMM_REGISTER_STAGED=1) on a MiniMind2 prefill
