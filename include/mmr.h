@@ -437,11 +437,15 @@ int mmr_batch_state_free(mmr_batch_state* state);
 /* batch, capacity (positions per sequence), steps run since the prompts; any may be NULL */
 int mmr_batch_state_info(const mmr_batch_state* state, int64_t* batch, int64_t* capacity, int64_t* steps);
 int mmr_batch_state_stream(const mmr_batch_state* state, mmr_stream_t* stream);
+/* Device bytes that the buffers of the prompts' passes hold (see mmr_batch_prefill). */
+int mmr_batch_state_prompt_bytes(const mmr_batch_state* state, uint64_t* device_bytes);
 /* tokens: the prompts concatenated; lengths[batch].  Fresh state only; advances
  * every sequence by max(lengths) positions (shorter prompts start generating
  * earlier): the tokens that all prompts have go through the prefill layers in
- * blocks of rows (their buffers are allocated here, on the first call), the
- * rest through steps. */
+ * passes of up to 4,096 rows, the rest through steps.  The passes' buffers (about
+ * 49 KB a row for MiniMind2) are allocated here and given back by the state's
+ * next synchronisation (mmr_batch_synchronize, the reads); where the device does
+ * not have the memory the passes are shorter, or all tokens go through steps. */
 int mmr_batch_prefill(const mmr_model* model, mmr_batch_state* state, const int32_t* tokens, const int64_t* lengths,
                       int64_t batch);
 int mmr_batch_decode(const mmr_model* model, mmr_batch_state* state, int64_t steps);

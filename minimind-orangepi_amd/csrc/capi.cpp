@@ -1282,6 +1282,13 @@ int mmr_batch_state_stream(const mmr_batch_state* state, mmr_stream_t* stream) {
   });
 }
 
+int mmr_batch_state_prompt_bytes(const mmr_batch_state* state, uint64_t* device_bytes) {
+  return guarded([&] {
+    require(state && device_bytes, "null argument");
+    *device_bytes = state->st.prompt_bytes();
+  });
+}
+
 int mmr_batch_prefill(const mmr_model* model, mmr_batch_state* state, const int32_t* tokens, const int64_t* lengths,
                       int64_t batch) {
   return guarded([&] {

@@ -77,11 +77,12 @@ struct BatchDeviceState {
   int32_t* staging = nullptr;  // pinned host
   int64_t staging_len = 0;
   hipStream_t stream = nullptr;
-  DeviceBuffer prompt_buf;     // h rows and the layer scratch of enqueue_prompt_rows
+  DeviceBuffer prompt_buf;     // h rows and the layer scratch of enqueue_prompt_rows, until the first synchronize
   std::map<int, hipGraphExec_t> graphs;
   bool use_graphs = true;
   bool prompt_tokenwise = false;  // prompts through the decode steps (comparison switch)
   int64_t prompt_rows = kPromptRows;
+  std::size_t prompt_limit = SIZE_MAX;  // bytes of prompt_buf
   bool register_staged = false;   // prompt GEMMs on the register-staged kernel only (comparison switch)
   // L2-warming blocks of the residual + norm launches (0 = none): the one
   // after the O projection loads gate_up and down, the one after down the
@@ -102,6 +103,7 @@ BatchState::BatchState(BatchState&&) noexcept = default;
 BatchState& BatchState::operator=(BatchState&&) noexcept = default;
 int64_t BatchState::batch() const { return device ? device->batch : 0; }
 int64_t BatchState::capacity() const { return device ? device->capacity : 0; }
+std::size_t BatchState::prompt_bytes() const { return device ? device->prompt_buf.bytes() : 0; }
 void* BatchState::stream() const { return device ? static_cast<void*>(device->stream) : nullptr; }
 
 namespace {
@@ -342,19 +344,32 @@ void enqueue_batch_step_kernels(const BatchDeviceState& s, int splits) {
 // as long as this many steps.
 constexpr int64_t kMinPromptRows = 4;
 
+std::size_t prompt_h_bytes(const BatchDeviceState& s, int64_t tokens) {
+  return Arena::round_up(static_cast<std::size_t>(s.batch * tokens * s.model->cfg.hidden_size) * sizeof(float));
+}
+
+// prompt_buf for passes over `count` tokens of every sequence: tokens of each
+// pass, equal passes of at most prompt_rows rows, or of half as many and so on
+// where the memory is not to be had; 0 if not even short ones.
+int64_t reserve_prompt_rows(BatchDeviceState& s, int64_t count) {
+  for (int64_t most = std::max<int64_t>(1, s.prompt_rows / s.batch);; most /= 2) {
+    const int64_t chunk = prefill_pass_rows(count, most);
+    const std::size_t bytes = prompt_h_bytes(s, chunk) + prefill_scratch_bytes(s.model->cfg, s.batch * chunk);
+    if (bytes <= s.prompt_limit && s.prompt_buf.try_reset(bytes)) return chunk;
+    if (most / 2 < kMinPromptRows) return 0;
+  }
+}
+
 // Tokens 0 .. count - 1 of every sequence into the KV pools through the
-// batched prefill layers: rows [sequence][token], in equal passes of at most
-// prompt_rows rows.
-// Nothing is predicted: the last layer stops after its keys and values.
-void enqueue_prompt_rows(BatchDeviceState& s, int64_t count) {
+// batched prefill layers: rows [sequence][token], `chunk` tokens of each
+// sequence at a time (prompt_buf holds that many).  Nothing is predicted: the
+// last layer stops after its keys and values.
+void enqueue_prompt_rows(BatchDeviceState& s, int64_t count, int64_t chunk) {
   const DeviceModel& m = *s.model;
   const auto& c = m.cfg;
-  const int64_t chunk = prefill_pass_rows(count, std::max<int64_t>(1, s.prompt_rows / s.batch));
-  const std::size_t h_bytes = Arena::round_up(static_cast<std::size_t>(s.batch * chunk * c.hidden_size) * sizeof(float));
-  s.prompt_buf.reset(h_bytes + prefill_scratch_bytes(c, s.batch * chunk));
   float* h = static_cast<float*>(s.prompt_buf.data());
-  PrefillScratch scratch =
-      carve_prefill_scratch(c, s.batch * chunk, static_cast<char*>(s.prompt_buf.data()) + h_bytes);
+  PrefillScratch scratch = carve_prefill_scratch(
+      c, s.batch * chunk, static_cast<char*>(s.prompt_buf.data()) + prompt_h_bytes(s, chunk));
   scratch.register_staged = s.register_staged;
   for (int64_t first = 0; first < count; first += chunk) {
     const int tokens = static_cast<int>(std::min(chunk, count - first));
@@ -437,6 +452,7 @@ BatchState LanguageModel::make_batch_state(int64_t batch, int64_t capacity, KvCa
   s->use_graphs = !(nog && nog[0] == '1');
   const char* pt = std::getenv("MMR_PREFILL_TOKENWISE");
   s->prompt_tokenwise = pt && pt[0] == '1';
+  s->prompt_limit = prefill_buffer_limit();
   if (const char* pc = std::getenv("MMR_PREFILL_CHUNK")) s->prompt_rows = std::max<int64_t>(1, std::atoll(pc));
   const char* rs = std::getenv("MMR_GEMM_REGISTER_STAGED");
   s->register_staged = rs && rs[0] == '1';
@@ -538,6 +554,16 @@ void LanguageModel::enqueue_batch_prefill(BatchState& state, const std::vector<s
   }
   if (longest > s.capacity) throw std::length_error("KV cache capacity exhausted");
   check_hip(hipStreamSynchronize(s.stream), "hipStreamSynchronize");
+  // All but the last token of the shortest prompt go through the prefill
+  // layers, for every sequence alike, so the sequences stay in lockstep; the
+  // steps take over where the first of them has to predict (no schedule needs
+  // fewer steps: the shortest prompt predicts one token in each of them).  A
+  // step reads all weights for one row of each sequence: 32 prompts of 192 to
+  // 256 tokens and 16 steps of MiniMind2 took 151 ms with every token in a
+  // step, 54 ms this way.
+  int64_t known = !s.prompt_tokenwise && shortest - 1 >= kMinPromptRows ? shortest - 1 : 0;
+  const int64_t chunk = known > 0 ? reserve_prompt_rows(s, known) : 0;
+  if (chunk == 0) known = 0;
   const int64_t stride = s.capacity + 1;
   std::memset(s.staging, 0, static_cast<std::size_t>(s.batch * stride) * sizeof(int32_t));
   int32_t* lens = s.staging + s.batch * stride;
@@ -549,20 +575,12 @@ void LanguageModel::enqueue_batch_prefill(BatchState& state, const std::vector<s
             "hipMemcpyAsync prompts");
   check_hip(hipMemcpyAsync(s.prompt_len, lens, s.batch * sizeof(int32_t), hipMemcpyHostToDevice, s.stream),
             "hipMemcpyAsync prompt lengths");
-  // All but the last token of the shortest prompt go through the prefill
-  // layers, for every sequence alike, so the sequences stay in lockstep; the
-  // steps take over where the first of them has to predict (no schedule needs
-  // fewer steps: the shortest prompt predicts one token in each of them).  A
-  // step reads all weights for one row of each sequence: 32 prompts of 192 to
-  // 256 tokens and 16 steps of MiniMind2 took 151 ms with every token in a
-  // step, 54 ms this way.
-  const int64_t known = !s.prompt_tokenwise && shortest - 1 >= kMinPromptRows ? shortest - 1 : 0;
   int32_t* pos = lens + s.batch;
   std::fill(pos, pos + s.batch, static_cast<int32_t>(known));
   check_hip(hipMemcpyAsync(s.pos, pos, s.batch * sizeof(int32_t), hipMemcpyHostToDevice, s.stream),
             "hipMemcpyAsync pos");
   if (known > 0) {
-    enqueue_prompt_rows(s, known);
+    enqueue_prompt_rows(s, known, chunk);
     state.steps = known;
   }
   for (int64_t i = known; i < longest; ++i) launch_batch_step(state);
@@ -581,6 +599,7 @@ void LanguageModel::synchronize(BatchState& state) const {
   int32_t* flag = s.staging + s.staging_len - 1;
   check_hip(hipMemcpyAsync(flag, s.err, sizeof(int32_t), hipMemcpyDeviceToHost, s.stream), "hipMemcpyAsync err");
   check_hip(hipStreamSynchronize(s.stream), "hipStreamSynchronize");
+  s.prompt_buf.reset(0);  // prompts come once in a state's life
   if (*flag != 0) throw std::runtime_error("device kernel reported an out-of-range position");
 }
 

@@ -76,6 +76,7 @@ struct BatchState {
   int64_t steps = 0;  // batched steps run since the prompts were set (host mirror)
   int64_t batch() const;
   int64_t capacity() const;  // positions per sequence
+  std::size_t prompt_bytes() const;  // held by the buffers of the prompts' passes
   void* stream() const;
   std::unique_ptr<BatchDeviceState> device;
 };

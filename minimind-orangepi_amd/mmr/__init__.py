@@ -191,6 +191,7 @@ _SIGS = {
     "mmr_batch_state_free": ([VP], C.c_int),
     "mmr_batch_state_info": ([VP, C.POINTER(I64), C.POINTER(I64), C.POINTER(I64)], C.c_int),
     "mmr_batch_state_stream": ([VP, C.POINTER(VP)], C.c_int),
+    "mmr_batch_state_prompt_bytes": ([VP, C.POINTER(C.c_uint64)], C.c_int),
     "mmr_batch_prefill": ([VP, VP, VP, VP, I64], C.c_int),
     "mmr_batch_decode": ([VP, VP, I64], C.c_int),
     "mmr_batch_synchronize": ([VP, VP], C.c_int),
@@ -999,6 +1000,13 @@ class BatchState:
         s = VP()
         check(_lib.mmr_batch_state_stream(self.handle, C.byref(s)))
         return s.value
+
+    @property
+    def prompt_bytes(self) -> int:
+        """Device bytes that the buffers of the prompts' passes hold, until the state is synchronized."""
+        n = C.c_uint64()
+        check(_lib.mmr_batch_state_prompt_bytes(self.handle, C.byref(n)))
+        return n.value
 
     def prefill(self, prompts) -> None:
         lengths = np.array([len(p) for p in prompts], np.int64)

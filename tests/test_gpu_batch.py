@@ -186,8 +186,10 @@ def test_batch_prompt_rows_take_many_rows_attention(gpu, monkeypatch, d, kv, bat
     rows = m.make_batch_state(batch, last, kvd)
     for st in (tok, rows):
         st.prefill(prompts)
+        assert (st.prompt_bytes > 0) is (st is rows)
         st.decode(4)
         st.synchronize()
+        assert st.prompt_bytes == 0  # given back
     for b in sorted({0, 1, batch // 2, batch - 1}):
         np.testing.assert_array_equal(rows.read_sequence(b, 0, last + 1), tok.read_sequence(b, 0, last + 1))
         assert rel_err(rows.read_logits(b), tok.read_logits(b)) < (1e-4 if kv == "f32" else 1e-3), b
@@ -213,6 +215,36 @@ def test_batch_prompt_rows_follow_the_switches(gpu, monkeypatch, switch, value):
     for b in range(5):
         np.testing.assert_array_equal(other.read_sequence(b, 0, 71), plain.read_sequence(b, 0, 71))
         assert rel_err(other.read_logits(b), plain.read_logits(b)) < 1e-5, b
+
+
+@pytest.mark.parametrize("megabytes,bitwise", [("0", True), ("1", False)])
+def test_batch_prompts_without_the_pass_buffers(gpu, monkeypatch, megabytes, bitwise):
+    # no memory for the passes' buffers: the prompts through the steps, bit for
+    # bit; 1 MB: shorter passes.  The state answers as ever.
+    mmr = gpu
+    print(f"[case] batch prompts with {megabytes} MB for passes", flush=True)
+    g = load_golden("mini")
+    m = synth_model(mmr, g)
+    rng = np.random.default_rng(3)
+    prompts = [[int(t) for t in rng.integers(0, g["config"]["vocab_size"], 302 + b)] for b in range(9)]
+    monkeypatch.setenv("MMR_PREFILL_TOKENWISE", "1")
+    tok = m.make_batch_state(9, 320, mmr.KV_F32)
+    monkeypatch.delenv("MMR_PREFILL_TOKENWISE")
+    monkeypatch.setenv("MMR_PREFILL_BUFFER_MB", megabytes)
+    few = m.make_batch_state(9, 320, mmr.KV_F32)
+    for st in (tok, few):
+        st.prefill(prompts)
+        assert st.prompt_bytes <= int(megabytes) << 20
+        st.decode(4)
+        st.synchronize()
+        st.decode(2)
+        st.synchronize()
+    for b in range(9):
+        np.testing.assert_array_equal(few.read_sequence(b, 0, 317), tok.read_sequence(b, 0, 317))
+        if bitwise:
+            np.testing.assert_array_equal(few.read_logits(b), tok.read_logits(b))
+        else:
+            assert rel_err(few.read_logits(b), tok.read_logits(b)) < 1e-4, b
 
 
 def test_batch_reproduces_reference_golden(gpu):
