@@ -365,10 +365,10 @@ void launch(const GemmArgs& g, hipStream_t s) {
   const dim3 grid((tiles + kXcds - 1) / kXcds * kXcds, 1, g.k_splits);  // x % 8 == 0: a tile's splits share an XCD
   if (g.k_splits > 1) {
     gemm_rows_kernel<kA, kStoreSplit><<<grid, kThreads, 0, s>>>(g);
-  } else if (g.swiglu) {
-    gemm_rows_kernel<kA, kSwiGlu><<<grid, kThreads, 0, s>>>(g);
-  } else if (g.residual) {
-    gemm_rows_kernel<kA, kResidual><<<grid, kThreads, 0, s>>>(g);
+  } else if (g.swiglu || g.residual) {
+    // Of planes, as the layers call it, or onto a caller's fp32 rows.
+    constexpr int kEpi = kA == kAPlanes ? kSwiGlu : kResidual;
+    gemm_rows_kernel<kA, kEpi><<<grid, kThreads, 0, s>>>(g);
   } else {
     gemm_rows_kernel<kA, kStore><<<grid, kThreads, 0, s>>>(g);
   }
@@ -426,7 +426,8 @@ bool gemm_many_rows(const GemmArgs& g) {
   const int64_t tiles = static_cast<int64_t>((g.m + kBM - 1) / kBM) * ((g.n + kBN - 1) / kBN);
   const bool enough = g.k_splits == 1 ? gemm_rows_unsplit(g.m, g.n, g.k) : g.k_splits == gemm_rows_splits(g.m, g.n, g.k);
   return enough && tiles < (1 << 30) && !g.register_staged && g.k % (2 * kBK) == 0 &&
-         (!g.a_hi || g.a_chunk == kSplitChunk) && (!g.swiglu || (g.n % 8 == 0 && g.ldc % 4 == 0)) &&
+         (!g.a_hi || (g.a_chunk == kSplitChunk && !g.residual)) &&
+         (!g.swiglu || (g.a_hi && g.n % 8 == 0 && g.ldc % 4 == 0)) &&
          (reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.a_hi) | reinterpret_cast<uintptr_t>(g.a_lo) |
           reinterpret_cast<uintptr_t>(g.w)) % 16 == 0 &&
          a_bytes < (int64_t{1} << 32) && w_bytes < (int64_t{1} << 32) && g.lda < (1 << 23);
