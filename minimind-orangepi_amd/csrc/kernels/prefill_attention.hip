@@ -82,7 +82,7 @@ __device__ __forceinline__ float sum16(const float (&p)[16]) {
 
 // The end of a block: the key ranges' (m, l) per query and O^T, as the lanes
 // of wave (s, hb) hold them, merge pairwise through `mrg`, and range 0's waves
-// write the rows.  The block has met since `mrg` was last read.
+// write the rows.
 template <int D, int HB>
 __device__ __forceinline__ void merge_and_write(const PrefillAttnArgs& a, f32x16 (&ot)[D / 32], float m_run,
                                                 float l_part, float* mrg, int s, int hb, int lane, int h, int b,
@@ -92,7 +92,7 @@ __device__ __forceinline__ void merge_and_write(const PrefillAttnArgs& a, f32x16
   const int qi = lane % 32, half = lane / 32;
 #pragma unroll
   for (int step = S / 2; step >= 1; step /= 2) {
-    if (step < S / 2) __syncthreads();  // the previous round's values have been read
+    __syncthreads();  // the stages (or the previous round's values) have been read
     if (s >= step && s < 2 * step) {
       float* dst = mrg + ((s - step) * HB + hb) * kMergeFloats;
 #pragma unroll
