@@ -444,8 +444,9 @@ int mmr_batch_state_prompt_bytes(const mmr_batch_state* state, uint64_t* device_
  * earlier): the tokens that all prompts have go through the prefill layers in
  * passes of up to 4,096 rows, the rest through steps.  The passes' buffers (about
  * 49 KB a row for MiniMind2) are allocated here and given back by the state's
- * next synchronisation (mmr_batch_synchronize, the reads); where the device does
- * not have the memory the passes are shorter, or all tokens go through steps. */
+ * next synchronisation (mmr_batch_synchronize, the reads), which then waits for
+ * the device as every hipFree does; where the device does not have the memory the
+ * passes are shorter, or all tokens go through steps. */
 int mmr_batch_prefill(const mmr_model* model, mmr_batch_state* state, const int32_t* tokens, const int64_t* lengths,
                       int64_t batch);
 int mmr_batch_decode(const mmr_model* model, mmr_batch_state* state, int64_t steps);

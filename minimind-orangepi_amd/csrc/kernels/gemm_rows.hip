@@ -35,19 +35,25 @@ __device__ __forceinline__ int chunk_pos(int row, int chunk) { return row * kRow
 
 // Block = 128 x 256 of C, 8 waves of 64 x 64 (2 x 2 fragments of 32 x 32), K
 // in stages of 64: W and pre-split A by direct loads (whole 128-byte lines),
-// fp32 A through registers, where it is split hi + lo.  Per k step of 16 the
-// products are v_mfma_f32_32x32x16_f16 of the hi and the lo plane.
+// fp32 A through registers, where it is split hi + lo under a scale per row and 64
+// columns (32 in K splits, whose A the layers would otherwise split per 32).  Per
+// k step of 16 the products are v_mfma_f32_32x32x16_f16 of the hi and the lo plane.
 //
-// What bounds it: LDS (a stage is 64 KB written and 192 KB read for 2,048
-// cycles of matrix products per SIMD) and, on real data, the clock, which the
-// products pull down (the same launch on degenerate data ran 10% faster).  The
-// 64 x 64 tiles of prefill.hip bring twice the bytes per product into LDS, and
-// read twice as many from it.  2,048 rows of fp32 A, W 4096 x 768: 57.7 ->
-// 36.2 us (447 -> 712 TFLOP/s of products); 4,096 rows 106 -> 67 us; pre-split
-// A, 6,000 rows: gate_up + SwiGLU 109 -> 85 us, QKV 39 -> 29 us.  (128 x 128
-// tiles of 4 waves, two blocks per CU: 101 and 36 us; 64 x 128 per wave with
-// one level of sums: 96 us and twice the error.)  K may be split over
-// gridDim.z (gemm_rows_splits).
+// What bounds it: no unit alone.  While a CU holds a block the matrix cores work
+// 40% of the time on fp32 A (51% on planes with SwiGLU), the vector unit 49%
+// (25%), LDS 27% (25%), and waves wait a third of theirs, most of it at the
+// stages' barriers; on fp32 A the split of A is done again by every column tile.
+// On real data the products also pull the clock down (the same launch on
+// degenerate data ran 10% faster).  The 64 x 64 tiles of prefill.hip bring twice
+// the bytes per product into LDS, and read twice as many from it.  2,048 rows of
+// fp32 A, W 4096 x 768: 55.6 us there, 33.8 here (463 -> 762 TFLOP/s of
+// products).  Tried before the scales per 64 and 128 columns, pre-split A, 6,000
+// rows (gate_up + SwiGLU 85 us, QKV 29; prefill.hip 109 and 39): 128 x 128 tiles
+// of 4 waves, two blocks per CU, 101 and 36; 64 x 128 per wave with one level of
+// sums, 96 and twice the error.  One scale for a whole row, or one that follows
+// its largest value so far, was no faster (2,048 rows 34.2 us) and lost the bits
+// of columns far smaller than others.  K may be split over gridDim.z
+// (gemm_rows_splits).
 template <int kA, int kEpi>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_kernel(GemmArgs g) {
   __shared__ __align__(16) char lds[kStages * kStageBytes];

@@ -277,7 +277,7 @@ hipError_t launch_qkv_postprocess(const QkvPostArgs& a, KvDtype kv, hipStream_t 
 // ------------------------------------------------------------- prefill ----
 // C[m][n] = (residual[m][n] +) sum_k A[m][k] * W[n][k]: A fp32 (row stride
 // lda), W fp16 row-major [n][k], C fp32 (row stride ldc); residual may alias
-// C.  fp32 matrix cores, fp32 accumulation.  k % 8 == 0, lda % 4 == 0.
+// C.  fp16 matrix cores on split A, fp32 accumulation.  k % 8 == 0, lda % 4 == 0.
 // A [rows][cols] as the GEMM's fp16 matrix cores take it: per row and
 // `chunk`-wide column chunk a power-of-two scale s (the chunk's max |a|
 // mapped into [2^14, 2^15)), hi = fp16(s a), lo = fp16(s a - hi), inv = 1 / s.

@@ -2,7 +2,8 @@
 // fp16 matrix cores (hi/lo split of the fp32 activations), per-row q/k norm +
 // RoPE + KV-cache write, interleaved SwiGLU rows, and causal attention over
 // the cache on the matrix cores (fp16 with hi/lo q and p for an fp16 cache,
-// fp32 for an fp32 cache).
+// fp32 for an fp32 cache).  For many rows gemm_rows.hip and
+// prefill_attention.hip (split operands for an fp32 cache too) take over.
 //
 // Replaces the reference's device prefill layer (run_dense_prefill_layer_device,
 // decoder_layer.cpp:661-734): device_matmul / device_matmul_add with batch =

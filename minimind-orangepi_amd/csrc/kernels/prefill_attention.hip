@@ -192,7 +192,8 @@ __device__ __forceinline__ bool block_not_finite(const f32x16 (&ot)[DT], float l
 // query of its tile (0 times it is NaN, also where the key is masked), and with
 // split operands every value under its scale.  Here it reaches what the formula
 // says: scores of -inf count for nothing, a value touches its own dim, and
-// queries before it stay as they are.  Wave: HB heads x queries s, s + S, ...;
+// queries before it stay as they are.  It takes some 50 to 100 times as long (6,000
+// rows with a NaN in key 0's value: fp16 0.16 -> 14 ms, fp32 0.31 -> 32).  Wave: HB heads x queries s, s + S, ...;
 // lane: a key of 64 for the scores, dims lane and lane + 64 for the values.
 template <typename KV, int D, int HB, bool kPool>
 __device__ void attend_rows_plainly(const PrefillAttnArgs& a, int s, int lane, int h, int b, int q0) {
@@ -277,7 +278,8 @@ __device__ void attend_rows_plainly(const PrefillAttnArgs& a, int s, int lane, i
 // log2(e) / sqrt(d) (folded into q), the softmax is base 2.
 //
 // What bounds it: the matrix cores (24 products of 32 cycles a tile and head
-// for d = 96) and, beside them, the softmax's vector instructions.  A wave
+// for d = 96; 46% of the time a CU holds a block) and, beside them, the softmax's
+// vector instructions (55%; LDS 13%).  A wave
 // alone leaves the matrix cores idle through its LDS reads, loads and
 // bookkeeping, so the products of tile i + 1's scores and tile i - 1's values
 // are formed while tile i's scores become probabilities, and the two waves of
@@ -547,9 +549,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // into the stage that the four heads share: a wave stages 8 rows of K and D / 4
 // dims of all 32 rows of V, so that each scale is its own to find.
 //
-// What bounds it: 36 products of 32 cycles a tile and head for d = 96 (1,152
-// cycles, where products of fp32 operands would take 6,144), and the splits' and
-// the softmax's vector instructions beside them.  prefill.hip's kernel / this
+// What bounds it: the splits' and the softmax's vector instructions (67% of the
+// time a CU holds a block, d = 96) beside 36 products of 32 cycles a tile and
+// head (37%; 1,152 cycles, where products of fp32 operands would take 6,144).  prefill.hip's kernel / this
 // one, 8 query heads on 2: d 96, 2,000 rows 118.9 / 89.3 us, 4,096 rows 398.1 /
 // 170.5, 3,000 rows after 1,111 keys 349.8 / 171.3; d 64 77.6 / 71.5, 248.3 /
 // 136.5, 222.4 / 137.6.  Error against 64 bits of each dimension, of its own

@@ -1,4 +1,4 @@
-"""GPU parity of the prefill path: the batched projection (fp32 matrix cores),
+"""GPU parity of the prefill path: the batched projection (split fp16 operands),
 the q/k norm + RoPE + KV-write rows, causal prefill attention, and the chunked
 model prefill against token-by-token decode.
 
@@ -56,7 +56,7 @@ def test_matmul_matches_fp64_and_oracle(gpu, oracle, batch, rows, cols):
 def test_matmul_many_rows_matches_fp64(gpu, batch, rows, cols, grow):
     # the 128 x 256 tiles (96 of them): a last row tile of 1 row, a last column
     # tile of 1 column, the shortest K, an odd number of 128-column chunks;
-    # rows whose values grow or shrink by 2^60 along K (the running row scale),
+    # rows whose values grow or shrink by 2^60 along K (a scale per 64 columns),
     # every row by another offset.  Against 64 bits, each row over its own
     # scale: the planes hold 22 bits of the row's largest values (2.4e-7), the
     # sums are fp32 over at most 1,408 products of like size (40 ulp at most).
@@ -503,8 +503,8 @@ def test_minimind2_ragged_chunks_match_tokenwise(gpu, monkeypatch, prompt_len):
 @pytest.mark.parametrize("prompt_len", [2305, 2500, 3500, 5000])
 def test_minimind2_long_passes_match_chunks(gpu, monkeypatch, prompt_len):
     # one pass of 2,500 rows and two of them (the many-rows GEMM for every
-    # projection, O and down in 3 K splits, QKV in 2; the many-rows attention
-    # after 2,500 cached rows), 2,305 (a last row tile of 1 row, K in uneven
+    # projection, O and down in 3 K splits, QKV in 2; the many-rows attention,
+    # also after 2,500 cached rows), 2,305 (a last row tile of 1 row, K in uneven
     # splits of 5, 5 and 6 chunks) and 3,500 (2 splits, QKV 1) against the
     # same prompt in 512-row chunks: same next token, logits within 1e-4 (fp16
     # K/V roundings of differently grouped fp32 sums, as in the tests below)
