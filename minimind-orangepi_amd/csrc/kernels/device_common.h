@@ -190,6 +190,19 @@ __device__ __forceinline__ void dma_load(const void* sbase, uint32_t voff, uint3
   }
 }
 
+// x = hi + lo in fp16, each rounded to nearest: 22 significant bits.  lo =
+// fp16(x - hi) is one instruction per value: hi * -1 + x, exact in fp32,
+// converted by v_fma_mix as it is written.  Lo is taken from hi's own bits: the
+// compiler may fuse a multiplication into one of two conversions of the same
+// value and not into the other, and the two then differ in a tie.
+using f32x2 = float __attribute__((ext_vector_type(2)));
+using f16x2 = _Float16 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, f16x2));
+  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(x0));
+  asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(x1));
+}
+
 // LDS byte address of a shared-memory pointer.
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const lds_byte*)p));

@@ -877,20 +877,13 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_attention_kernel
     for (int j = 0; j < D / 32; ++j) {
       const float4 x0 = *reinterpret_cast<const float4*>(qsrc + 32 * j + 8 * kq);
       const float4 x1 = *reinterpret_cast<const float4*>(qsrc + 32 * j + 8 * kq + 4);
-      float x[8] = {x0.x * qscale, x0.y * qscale, x0.z * qscale, x0.w * qscale,
-                    x1.x * qscale, x1.y * qscale, x1.z * qscale, x1.w * qscale};
-      f16x8 hv, lv;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        // x rounded, for both planes: with the product fused into one of the
-        // two conversions, a tie gave a hi plane one unit off the one that lo
-        // was taken from (1e-4 of a score, in 1 of some 10^4 elements).
-        asm("" : "+v"(x[e]));
-        hv[e] = static_cast<_Float16>(x[e]);
-        lv[e] = static_cast<_Float16>(x[e] - static_cast<float>(hv[e]));
-      }
-      qh[j] = __builtin_bit_cast(uint4, hv);
-      ql[j] = __builtin_bit_cast(uint4, lv);
+      uint32_t hi[4], lo[4];
+      split2(x0.x * qscale, x0.y * qscale, hi[0], lo[0]);
+      split2(x0.z * qscale, x0.w * qscale, hi[1], lo[1]);
+      split2(x1.x * qscale, x1.y * qscale, hi[2], lo[2]);
+      split2(x1.z * qscale, x1.w * qscale, hi[3], lo[3]);
+      qh[j] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+      ql[j] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
     }
   } else {
 #pragma unroll

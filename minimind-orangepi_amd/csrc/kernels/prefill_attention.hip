@@ -12,8 +12,6 @@
 namespace mmr {
 namespace {
 
-using f32x2 = float __attribute__((ext_vector_type(2)));
-using f16x2 = _Float16 __attribute__((ext_vector_type(2)));
 using f32x4 = float __attribute__((ext_vector_type(4)));
 using f32x16 = float __attribute__((ext_vector_type(16)));
 using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
@@ -55,14 +53,7 @@ __device__ __forceinline__ float half_swap_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// x = hi + lo in fp16, each rounded to nearest: 22 significant bits.  lo =
-// fp16(x - hi) is one instruction per value: hi * -1 + x, exact in fp32,
-// converted by v_fma_mix as it is written.
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
-  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, f16x2));
-  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(x0));
-  asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(x1));
-}
+// Eight values split hi + lo (split2).
 __device__ __forceinline__ void split8(const float* x, f16x8& hi, f16x8& lo) {
   uint32_t h[4], l[4];
 #pragma unroll
