@@ -560,7 +560,7 @@ void LanguageModel::enqueue_batch_prefill(BatchState& state, const std::vector<s
   // fewer steps: the shortest prompt predicts one token in each of them).  A
   // step reads all weights for one row of each sequence: 32 prompts of 192 to
   // 256 tokens and 16 steps of MiniMind2 took 151 ms with every token in a
-  // step, 54 ms this way.
+  // step, 53 ms this way.
   int64_t known = !s.prompt_tokenwise && shortest - 1 >= kMinPromptRows ? shortest - 1 : 0;
   const int64_t chunk = known > 0 ? reserve_prompt_rows(s, known) : 0;
   if (chunk == 0) known = 0;
