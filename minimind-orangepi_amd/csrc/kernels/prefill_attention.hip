@@ -548,7 +548,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // 136.5, 222.4 / 137.6.  Error against 64 bits of each dimension, of its own
 // largest value (d 96, 2,000 rows after 2,000 keys): 2.0e-6 / 1.1e-6; with V's
 // dimensions spread over 2^16 1.9e-6 / 1.1e-6, its keys over 2^20 2.2e-6 /
-// 1.8e-6, q and (inversely) k over 2^8 1.9e-6 / 1.2e-6.  (A tile's values are
+// 1.8e-6, q's dimensions and (inversely) k's over 2^8 1.9e-6 / 1.2e-6, over 2^20
+// 1.9e-6 / 1.3e-6, but over 2^24 1.8e-6 / 1.9e-5.  (A tile's values are
 // summed before they meet the long sums: added product by product, 3,000 rows
 // after 3,000 keys had 5.9e-7 of the largest value against 3.4e-7.  Under one V
 // scale per 8 keys and all dims, dimensions 2^-20 of the others' size had 8.7e-6
